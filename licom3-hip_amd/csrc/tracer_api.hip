@@ -200,12 +200,6 @@ int plan_step(licom_ctx *c, const licom_fields *f, int &flags, bool &split, cons
         set_error("boundary_restore=1 needs the restore field");
         return LICOM_EINVAL;
     }
-    // The fused k-march stages planes in 16-byte chunks: it needs an even imt
-    // and 16-byte aligned at, atb, ws and akt; other layouts take the
-    // per-stage kernels (same results).
-    const uintptr_t al = reinterpret_cast<uintptr_t>(f->at) | reinterpret_cast<uintptr_t>(f->atb) |
-                         reinterpret_cast<uintptr_t>(f->ws) | reinterpret_cast<uintptr_t>(f->akt);
-    if (c->imt % 2 != 0 || (al & 15) != 0) flags |= LICOM_STEP_STAGED;
     if (flags & LICOM_STEP_ICESNOW) {
         if (!c->qice) {
             set_error("LICOM_STEP_ICESNOW needs licom_tracer_set_icesnow first");
@@ -412,6 +406,7 @@ int licom_tracer_create(const licom_grid *G, const licom_params *P, licom_ctx **
     rc = rc ? rc : plan_scratch(&s.uw, n3);
     rc = rc ? rc : plan_scratch(&s.vs, n3);
     rc = rc ? rc : plan_scratch(&s.ori, 2 * n3);
+    if (P->adv == LICOM_ADV_TSPAS) rc = rc ? rc : plan_scratch(&s.flags, 2 * n3);
     rc = rc ? rc : plan_scratch(&s.mix_count, 2);
     rc = rc ? rc : place_parts();
     if (rc) {
@@ -435,11 +430,10 @@ int licom_tracer_step(licom_ctx *c, const licom_fields *f, const licom_diag *d, 
     int rc;
     if (run & LICOM_STEP_STAGED) {
         // scratch of the per-stage kernels, allocated on first use
-        if (!c->s.flags) {
-            rc = scratch(c, &c->s.flags, 2 * c->n3);
-            if (!rc && c->p.hmix == LICOM_HMIX_DEL4) rc = scratch(c, &c->s.d2tk, 2 * c->n3);
-            if (rc) return rc;
-        }
+        if (!c->s.flags)
+            if ((rc = scratch(c, &c->s.flags, 2 * c->n3))) return rc;
+        if (!c->s.d2tk && c->p.hmix == LICOM_HMIX_DEL4)
+            if ((rc = scratch(c, &c->s.d2tk, 2 * c->n3))) return rc;
         rc = launch_step_simple(c, f, d, run);
     } else {
         rc = launch_step_fused(c, f, d, run, c->s);

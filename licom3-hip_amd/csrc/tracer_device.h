@@ -21,7 +21,9 @@ __device__ __forceinline__ double wk(double uf, double ul, double oncc) {
 // s/n = j+-1, u/d = k-+1), Ue/Uw the west-face velocities at i+1 and i,
 // Vs/Vn the south-face velocities at j and j-1, Wk/Wb the vertical velocity at
 // the top and bottom of the cell, D1..D4 the face metric products
-// htw*hun (i+1), htw*hun (i), hts*hue (j), hts*hue (j-1).
+// htw*hun (i+1), htw*hun (i), hts*hue (j), hts*hue (j-1), oz, ot, ot1 the
+// level's odzp[k], odzt[k] and odzt[k+1] (ot at k = 0 and ot1 at k = km-1 are
+// not used).
 struct PTerms {
     double x0, y0, xy1, xy2, xy3, xy4, c1, c2, za, zb1, zb2, zc;
 };
@@ -31,20 +33,20 @@ __device__ __forceinline__ void pterms_cheap(double Tc, double Te, double Tw, do
                                              double Tn, double Tu, double Td, double Ue,
                                              double Uw, double Vs, double Vn, double Wk,
                                              double Wb, double tr, int k, int km,
-                                             const double *odzp, PTerms &t) {
+                                             double oz, PTerms &t) {
     t.x0 = (Te + Tc) * Ue * tr - (Tc + Tw) * Uw * tr;
     t.y0 = ((Ts + Tc) * Vs - (Tc + Tn) * Vn) * tr;
     t.c1 = -Tc * (Ue - Uw) * tr * 2.0;
     t.c2 = -Tc * (Vs - Vn) * tr * 2.0;
     if (k == 0) {
-        t.za = -0.5 * odzp[0] * Wb * (Td + Tc);
-        t.zc = odzp[0] * Tc * Wb;
+        t.za = -0.5 * oz * Wb * (Td + Tc);
+        t.zc = oz * Tc * Wb;
     } else if (k == km - 1) {
-        t.za = 0.5 * odzp[k] * Wk * (Tc + Tu);
-        t.zc = -odzp[k] * Tc * Wk;
+        t.za = 0.5 * oz * Wk * (Tc + Tu);
+        t.zc = -oz * Tc * Wk;
     } else {
-        t.za = 0.5 * odzp[k] * Wk * (Tc + Tu) - 0.5 * odzp[k] * Wb * (Tc + Td);
-        t.zc = -odzp[k] * Tc * (Wk - Wb);
+        t.za = 0.5 * oz * Wk * (Tc + Tu) - 0.5 * oz * Wb * (Tc + Td);
+        t.zc = -oz * Tc * (Wk - Wb);
     }
 }
 
@@ -53,7 +55,7 @@ __device__ __forceinline__ void pterms_lw(double Tc, double Te, double Tw, doubl
                                           double Tu, double Td, double Ue, double Uw, double Vs,
                                           double Vn, double Wk, double Wb, double tr, double D1,
                                           double D2, double D3, double D4, int k, int km,
-                                          const double *odzp, const double *odzt, double dts,
+                                          double oz, double ot, double ot1, double dts,
                                           PTerms &t) {
     t.xy1 = -dts * (Te - Tc) * 2.0 * tr * Ue * Ue / D1;
     t.xy2 = dts * (Tc - Tw) * 2.0 * tr * Uw * Uw / D2;
@@ -61,13 +63,13 @@ __device__ __forceinline__ void pterms_lw(double Tc, double Te, double Tw, doubl
     t.xy4 = dts * (Tc - Tn) * 2.0 * tr * Vn * Vn / D4;
     if (k == 0) {
         t.zb1 = 0.0;
-        t.zb2 = 0.5 * odzp[0] * Wb * Wb * odzt[1] * (Tc - Td) * dts;
+        t.zb2 = 0.5 * oz * Wb * Wb * ot1 * (Tc - Td) * dts;
     } else if (k == km - 1) {
-        t.zb1 = -0.5 * odzp[k] * Wk * Wk * odzt[k] * (Tu - Tc) * dts;
+        t.zb1 = -0.5 * oz * Wk * Wk * ot * (Tu - Tc) * dts;
         t.zb2 = 0.0;
     } else {
-        t.zb1 = -0.5 * odzp[k] * Wk * Wk * odzt[k] * (Tu - Tc) * dts;
-        t.zb2 = 0.5 * odzp[k] * Wb * Wb * odzt[k + 1] * (Tc - Td) * dts;
+        t.zb1 = -0.5 * oz * Wk * Wk * ot * (Tu - Tc) * dts;
+        t.zb2 = 0.5 * oz * Wb * Wb * ot1 * (Tc - Td) * dts;
     }
 }
 
@@ -75,11 +77,11 @@ __device__ __forceinline__ void pterms(double Tc, double Te, double Tw, double T
                                        double Tu, double Td, double Ue, double Uw, double Vs,
                                        double Vn, double Wk, double Wb, double tr, double D1,
                                        double D2, double D3, double D4, int k, int km,
-                                       const double *odzp, const double *odzt, double dts,
+                                       double oz, double ot, double ot1, double dts,
                                        PTerms &t) {
-    pterms_cheap(Tc, Te, Tw, Ts, Tn, Tu, Td, Ue, Uw, Vs, Vn, Wk, Wb, tr, k, km, odzp, t);
-    pterms_lw(Tc, Te, Tw, Ts, Tn, Tu, Td, Ue, Uw, Vs, Vn, Wk, Wb, tr, D1, D2, D3, D4, k, km, odzp,
-              odzt, dts, t);
+    pterms_cheap(Tc, Te, Tw, Ts, Tn, Tu, Td, Ue, Uw, Vs, Vn, Wk, Wb, tr, k, km, oz, t);
+    pterms_lw(Tc, Te, Tw, Ts, Tn, Tu, Td, Ue, Uw, Vs, Vn, Wk, Wb, tr, D1, D2, D3, D4, k, km, oz,
+              ot, ot1, dts, t);
 }
 
 // Predictor value at00 (tracer.cpp:410-414).
@@ -103,7 +105,7 @@ struct CFAdv {
 __device__ __forceinline__ CFAdv adv_cf(int scheme, double Tc, double Te, double Tw, double Ts,
                                         double Tn, double Tu, double Td, double Ue, double Uw,
                                         double Vs, double Vn, double Wk, double Wb, double tr, int k,
-                                        int km, const double *odzp) {
+                                        int km, double oz) {
     CFAdv r;
     if (scheme == LICOM_ADV_CENTERED) {
         const double a = (-Uw * (Tc - Tw) - Ue * (Te - Tc) - Vs * (Ts - Tc) - Vn * (Tc - Tn)) * tr;
@@ -119,13 +121,13 @@ __device__ __forceinline__ CFAdv adv_cf(int scheme, double Tc, double Te, double
             const double z2 = Wb * (Tc - Td);
             z = z1 + z2;
         }
-        r.vz = 0.5 * odzp[k] * z;
-        r.adv = a - 0.5 * odzp[k] * z;
+        r.vz = 0.5 * oz * z;
+        r.adv = a - 0.5 * oz * z;
     } else {
         const double a = (-Uw * (Tc + Tw) + Ue * (Te + Tc) - Vn * (Tc + Tn) + Vs * (Ts + Tc)) * tr;
         const double z1 = (k == 0) ? 0.0 : Wk * (Tu + Tc) * 0.5;
         const double z2 = (k == km - 1) ? 0.0 : Wb * (Tc + Td) * 0.5;
-        r.adv = a - odzp[k] * (z2 - z1);
+        r.adv = a - oz * (z2 - z1);
         r.hx = r.hy = r.vz = 0.0;
     }
     return r;

@@ -1,6 +1,6 @@
 // tracer_fused.hip -- production path of the FP64 tracer step on gfx950.
 //
-// Four 3-D passes per step instead of the reference's ~21 launches per
+// Five 3-D passes per step instead of the reference's ~21 launches per
 // tracer (plus the 2-D surface, SSSNORM and halo kernels that the staged
 // path in tracer_kernels.hip shares):
 //
@@ -9,14 +9,9 @@
 //                  the barotropic-corrected velocity (upwell_2,
 //                  operators_div) and the continuity w (upwell_3/4), the
 //                  divergence profile held in registers.
-//   k_march        one four-wave workgroup per 16x12 tile of columns and
-//                  tracer, marching k top to bottom.  Waves 0-2 own the tile,
-//                  wave 3 the 56-cell ring the limiter and del4 read around
-//                  it; wave 3 also streams the planes of at, atb and the
-//                  velocities (tile plus a 2-cell halo) straight into LDS a
-//                  level ahead.  The tspas predictor of level k+1 feeds the
-//                  limiter of level k through LDS flag planes; the del4 first
-//                  pass stays in LDS.  Writes the explicit update (tracer_8's
+//   k_flags        tspas predictor and limiter flag of every cell (one byte)
+//   k_update       limited fluxes, horizontal mixing, shortwave and explicit
+//                  vertical diffusion.  Writes the explicit update (tracer_8's
 //                  vtl) and the advective / vertical-diffusion diagnostics.
 //   k_solve<KM>    two lanes per column (T and S): the implicit vertical
 //                  diffusion (invtrit) with checkpointed elimination
@@ -28,6 +23,9 @@
 // Arithmetic is shared with the per-stage kernels through tracer_device.h,
 // so both paths give identical bits.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <type_traits>
 
 #include "tracer_device.h"
 #include "tracer_internal.h"
@@ -191,532 +189,574 @@ __global__ __launch_bounds__(256) void k_prelude_col(KGrid g, KPar p, const doub
     }
 }
 
-// --------------------------------------------------------------- march
-constexpr int BX = 16, BY = 12;                 // interior tile (one lane per column)
-constexpr int PX = BX + 2, PY = BY + 2;         // tile + 1-cell ring (predictor, d2tk)
-constexpr int RX = BX + 4, RY = BY + 4;         // tile + 2-cell halo (staged planes)
-constexpr int NOWN = BX * BY;                   // 192 tile lanes: waves 0-2
-constexpr int NRING = 2 * (BX + BY);            // 56 ring cells: wave 3 (the ring's
-                                                // corners are never read)
-constexpr int NT = 256;                         // four waves
-static_assert(NOWN == 192 && NRING <= 64, "three tile waves and one ring wave");
-constexpr int NP = PX * PY, NR = RX * RY;
-// Staged planes are loaded LA levels ahead of the phase that first reads
-// them: at and ws are issued for level k+LA+2 at the start of P(k), the face
-// velocities, atb and akt for level k+LA+1.  LDS slots per array follow.
-constexpr int LA = 2;
-constexpr int NAT = LA + 3, NW = LA + 3, NUV = LA + 2, NB = LA + 2;
-// direct-to-LDS instructions the staging wave issues per level
-constexpr int DMA_ATW = 2 * ((NR / 2 + 63) / 64);          // at, ws
-constexpr int DMA_UVBA = 3 * ((NR / 2 + 63) / 64) + 2;     // u, v, atb + akt
+// --------------------------------------------------- limiter flags and update
+// Replaces a march of 16 x 12 tiles whose planes a fourth wave staged in LDS
+// (two barriers a level, two workgroups per CU: bound by the latency of its
+// level loop, 7.03 ms at 1800 x 1151 x 55, 71 us at 128 x 96 x 30; now 6.5 ms
+// and 31 us, k_flags bound by its ~200 FP64 instructions a cell and k_update
+// by its 11 + 8 planes of HBM traffic, 4.2 TB/s).
+// Neither kernel carries anything from one level to the next but values it
+// has already loaded, so a column is cut into chunks of levels and every
+// (chunk, run of cells, tracer) is a workgroup of its own.
+//
+// Each lane takes two consecutive cells of the plane, whatever the row
+// length, and neighbours along i come from the lanes beside it (DPP): the
+// vector cache handles a 16-byte access of a wave in the same 16 cycles as an
+// 8-byte one, and with one cell per lane (and so e and w loads of their own)
+// its access rate, not HBM, bounded the kernels.  A wave's first and last
+// lane only feed their neighbours: 124 of its 128 cells are its own.
+constexpr int kWaveCells = 124;
 
-struct MarchArgs {
-    const double *at, *atb, *akt, *uw, *vs, *ws, *stf_n, *err_norm2, *swv, *restore;
-    double *ori, *ax, *ay, *az, *dz, *pen;
+struct FlatGrid {
+    int first, last;  // cells [first, last) of the plane
+    int nch, kc;      // chunks of a column, levels per chunk
+    int total, per;   // workgroups, and workgroups per XCD
+};
+
+// Whole columns, where those give the 256 CUs four workgroups each (smaller
+// chunks read the levels around them again: at 1800 x 1151 x 55 chunks of 55,
+// 28, 14 and 7 levels took 7.3, 7.7, 8.1 and 8.7 ms for both kernels), and
+// otherwise as many chunks as that takes, of two levels at least.
+inline FlatGrid flat_grid(int first, int last, int km) {
+    const int nb = (last - first + 4 * kWaveCells - 1) / (4 * kWaveCells);
+    int nch = (1024 + 2 * nb - 1) / (2 * nb);
+    const int kc = std::max((km + nch - 1) / nch, 2);
+    nch = (km + kc - 1) / kc;
+    const int total = 2 * nb * nch;
+    return FlatGrid{first, last, nch, kc, total, (total + 7) / 8};
+}
+
+// Block -> (tracer, chunk, block of the plane): the two tracers of one place,
+// then its chunks, run next to each other, and the hardware's round-robin deal of blocks to
+// the eight XCDs is undone, so that each XCD's L2 sees a run of neighbouring
+// blocks, whose rows and face velocities they share.
+__device__ __forceinline__ bool flat_block(const FlatGrid &f, int &n, int &blk, int &k0) {
+    const int b = (int)blockIdx.x, L = (b & 7) * f.per + (b >> 3);
+    if (L >= f.total) return false;
+    n = L & 1;
+    const int h = L >> 1;
+    blk = h / f.nch;
+    k0 = (h - blk * f.nch) * f.kc;
+    return true;
+}
+
+// First of this lane's two cells; it may lie outside the plane for lanes
+// that own none of their cells.
+__device__ __forceinline__ int lane_cell(const FlatGrid &f, int blk) {
+    const int wave = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63);
+    return f.first + (blk * 4 + wave) * kWaveCells + 2 * (lane - 1);
+}
+
+// Two cells of a plane at byte offset `off`: the plane's address is the same
+// in every lane, so an access needs one 32-bit address register.
+struct D2 {
+    double v[2];
+};
+typedef double licom_d2 __attribute__((ext_vector_type(2), aligned(8)));
+typedef double licom_d2a __attribute__((ext_vector_type(2)));
+typedef uint16_t licom_u16 __attribute__((aligned(1)));
+__device__ __forceinline__ D2 ld2(const double *plane, uint32_t off) {
+    const licom_d2 x = *reinterpret_cast<const licom_d2 *>(reinterpret_cast<const char *>(plane) + off);
+    return D2{{x.x, x.y}};
+}
+__device__ __forceinline__ uint32_t ldf2(const uint8_t *plane, uint32_t off) {
+    return *reinterpret_cast<const licom_u16 *>(plane + off);
+}
+// Stores of the cells that a0 and a1 mark.  Non-temporal: nothing on this
+// path reads them again before the caches have turned over (k_update 5.22 ->
+// 5.02 ms at 1800 x 1151 x 55, 98 -> 82 us at 225 x 145 x 55).
+__device__ __forceinline__ void st2(double *plane, uint32_t off, const double (&x)[2], bool a0, bool a1) {
+    char *p = reinterpret_cast<char *>(plane) + off;
+    if (a0 && a1) {
+        __builtin_nontemporal_store(licom_d2{x[0], x[1]}, reinterpret_cast<licom_d2 *>(p));
+    } else if (a0 || a1) {
+        *reinterpret_cast<double *>(p + (a0 ? 0 : 8)) = a0 ? x[0] : x[1];
+    }
+}
+
+// Value of the lane before / after this one (DPP wave shift).
+template <int CTRL>
+__device__ __forceinline__ int dpp(int x) {
+    return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL>
+__device__ __forceinline__ double dppd(double x) {
+    const licom_v2i v = __builtin_bit_cast(licom_v2i, x);
+    return __builtin_bit_cast(double, licom_v2i{dpp<CTRL>(v.x), dpp<CTRL>(v.y)});
+}
+constexpr int kFromPrev = 0x138, kFromNext = 0x130;   // wave_shr:1, wave_shl:1
+
+// West and east neighbours of a lane's two cells.
+__device__ __forceinline__ D2 west(const D2 &x) { return D2{{dppd<kFromPrev>(x.v[1]), x.v[0]}}; }
+__device__ __forceinline__ D2 east(const D2 &x) { return D2{{x.v[1], dppd<kFromNext>(x.v[0])}}; }
+
+// Runs level(position, k) for the levels [k0, k1): position 0 is the surface
+// level, 2 the deepest and 1 any other, compiled apart so that the middle
+// levels are one run of instructions without branches.
+template <class F>
+__device__ __forceinline__ void march_levels(int k0, int k1, int km, F &&level) {
+    int k = k0;
+    if (k == 0) level(std::integral_constant<int, 0>{}, k++);
+    for (const int e = min(k1, km - 1); k < e; ++k) level(std::integral_constant<int, 1>{}, k);
+    if (k < k1) level(std::integral_constant<int, 2>{}, k);
+}
+
+// Byte offsets of the lane's cells and of those dj rows away, kept inside
+// the plane (a lane that owns a cell never has its offsets clamped).
+__device__ __forceinline__ int clamp_cell(int p, int n2) { return min(max(p, 0), n2 - 2); }
+
+// Keeps the compiler from forming plane + offset once per array outside the
+// level loop: 20 64-bit lane addresses, which spill, in place of scalar plane
+// addresses and one shared offset.
+__device__ __forceinline__ void fresh(uint32_t &off) { asm("" : "+v"(off)); }
+
+// Face products of the tspas terms: htw*hun at the west faces of the two
+// cells and of the one after them, hts*hue at their south and north faces.
+struct Faces {
+    double dx[3], ds[2], dn[2], tr[2];
+};
+__device__ __forceinline__ Faces load_faces(const KGrid &g, int pc, int pn) {
+    Faces f;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        f.tr[e] = g.tarea_r[pc + e];
+        f.dx[e] = g.htw[pc + e] * g.hun[pc + e];
+        f.ds[e] = g.hts[pc + e] * g.hue[pc + e];
+        f.dn[e] = g.hts[pn + e] * g.hue[pn + e];
+    }
+    f.dx[2] = dppd<kFromNext>(f.dx[0]);
+    return f;
+}
+
+// tspas predictor and limiter flag (advection_tracer_2, tracer.cpp:311-545),
+// one byte per cell, of every cell off the outermost rows and columns (the
+// outermost columns get bytes that nothing reads).
+__global__ __launch_bounds__(256, 4) void k_flags(KGrid g, double dts, const double *__restrict__ at,
+                                                  const double *__restrict__ uw, const double *__restrict__ vs,
+                                                  const double *__restrict__ ws, uint8_t *__restrict__ flags,
+                                                  const double *__restrict__ odzp, const double *__restrict__ odzt,
+                                                  FlatGrid fg) {
+    int n, blk, k0;
+    if (!flat_block(fg, n, blk, k0)) return;
+    const int imt = g.imt, km = g.km, n2 = imt * g.jmt, lane = (int)threadIdx.x & 63;
+    const int p = lane_cell(fg, blk);
+    const int pc = clamp_cell(p, n2), pn = clamp_cell(p - imt, n2), ps = clamp_cell(p + imt, n2);
+    uint32_t bc = 8u * (uint32_t)pc, bn = 8u * (uint32_t)pn, bs = 8u * (uint32_t)ps;
+    const bool own = lane >= 1 && lane <= 62;
+    const bool own0 = own && p < fg.last, own1 = own && p + 1 < fg.last;
+    const double *T = at + (size_t)n * n2 * km;
+    uint8_t *F = flags + (size_t)n * n2 * km;
+    const Faces fc = load_faces(g, pc, pn);
+    int kc[4], kn[2], ks[2];     // wet levels: cells -1..2, and the rows beside
+    kc[1] = g.kmt[pc];
+    kc[2] = g.kmt[pc + 1];
+    kc[0] = dpp<kFromPrev>(kc[2]);
+    kc[3] = dpp<kFromNext>(kc[1]);
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        kn[e] = g.kmt[pn + e];
+        ks[e] = g.kmt[ps + e];
+    }
+    const int k1 = min(k0 + fg.kc, km);
+    const size_t o0 = (size_t)k0 * n2;
+    D2 Tu{}, Tc = ld2(T + o0, bc), Wk = ld2(ws + o0, bc);
+    if (k0 > 0) Tu = ld2(T + o0 - n2, bc);
+    march_levels(k0, k1, km, [&](auto pos, int K) {
+        constexpr bool top = pos == 0, bot = pos == 2;
+        const double oz = odzp[K], ot = odzt[K], ot1 = bot ? 0.0 : odzt[K + 1];
+        const size_t o = (size_t)K * n2;
+        fresh(bc);
+        fresh(bn);
+        fresh(bs);
+        const D2 Tn = ld2(T + o, bn), Ts = ld2(T + o, bs);
+        const D2 U = ld2(uw + o, bc), Vs = ld2(vs + o, bc), Vn = ld2(vs + o, bn);
+        D2 Td{}, Wb{};
+        if constexpr (!bot) {
+            Td = ld2(T + o + n2, bc);
+            Wb = ld2(ws + o + n2, bc);
+        }
+        const D2 Tw = west(Tc), Te = east(Tc), Ue = east(U);
+        uint32_t fl = 0;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const double tc = Tc.v[e];
+            dev::PTerms t;
+            dev::pterms(tc, Te.v[e], Tw.v[e], Ts.v[e], Tn.v[e], Tu.v[e], Td.v[e], Ue.v[e], U.v[e], Vs.v[e], Vn.v[e],
+                        Wk.v[e], Wb.v[e], fc.tr[e], fc.dx[e + 1], fc.dx[e], fc.ds[e], fc.dn[e], top ? 0 : 1, bot ? 2 : 3, oz, ot, ot1, dts, t);
+            const double a00 = dev::predictor(t, tc, dts);
+            // 7-point bounds with land masked to -+1e10 (tracer.cpp:416-545)
+            const double lo = -1.0e10, hi = 1.0e10;
+            const int kz = kc[e + 1];
+            double mx = kz > K ? tc : lo, mn = kz > K ? tc : hi;
+            auto bound = [&](bool wet, double v) {
+                mx = fmax(mx, wet ? v : lo);
+                mn = fmin(mn, wet ? v : hi);
+            };
+            bound(kn[e] > K, Tn.v[e]);
+            bound(ks[e] > K, Ts.v[e]);
+            bound(kc[e] > K, Tw.v[e]);
+            bound(kc[e + 2] > K, Te.v[e]);
+            if constexpr (!top) bound(kz > K - 1, Tu.v[e]);
+            if constexpr (!bot) bound(kz > K + 1, Td.v[e]);
+            fl |= (uint32_t)(a00 > mx || a00 < mn) << (8 * e);
+        }
+        const uint32_t fc8 = bc >> 3;
+        if (own1) *reinterpret_cast<licom_u16 *>(F + o + fc8) = (uint16_t)fl;
+        else if (own0) F[o + fc8] = (uint8_t)fl;
+        Tu = Tc;
+        Tc = Td;
+        Wk = Wb;
+    });
+}
+
+// del2 stencil of a lane's two cells in one row (DTN..DTW).  load_wet gives
+// for each of the two, a byte each (n, s, e, w from the low end), the number
+// of levels at which it and that neighbour are both wet.
+struct Del2 {
+    D2 dn, ds, de, dw;
+};
+__device__ __forceinline__ void load_wet(const KGrid &g, int pc, int pn, int ps, uint32_t (&wet)[2]) {
+    const int a = g.kmt[pc], b = g.kmt[pc + 1];
+    const int w = dpp<kFromPrev>(b), z = dpp<kFromNext>(a);
+    const int kz[2] = {a, b}, kw[2] = {w, a}, ke[2] = {b, z};
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+        wet[e] = (uint32_t)min(kz[e], g.kmt[pn + e]) | (uint32_t)min(kz[e], g.kmt[ps + e]) << 8 |
+                 (uint32_t)min(kz[e], ke[e]) << 16 | (uint32_t)min(kz[e], kw[e]) << 24;
+}
+
+// cc * X + sum of the wet neighbours' terms (tracer.cpp:1165-1180, 1249-1286)
+__device__ __forceinline__ double del2(const Del2 &m, uint32_t wet, int e, uint32_t k, double Xc, double Xn, double Xs,
+                                       double Xe, double Xw) {
+    double h = 0.0, cc = 0.0;
+    if (k < (wet & 255u)) { h += m.dn.v[e] * Xn; cc -= m.dn.v[e]; }
+    if (k < (wet >> 8 & 255u)) { h += m.ds.v[e] * Xs; cc -= m.ds.v[e]; }
+    if (k < (wet >> 16 & 255u)) { h += m.de.v[e] * Xe; cc -= m.de.v[e]; }
+    if (k < (wet >> 24)) { h += m.dw.v[e] * Xw; cc -= m.dw.v[e]; }
+    return cc * Xc + h;
+}
+
+struct UpdateArgs {
+    const double *stf_n, *err_norm2, *swv, *restore;
+    double *ax, *ay, *az, *dz, *pen;
     uint8_t *flags_out;   // the limiter flag of every physical cell, or NULL
-    int ntx, ntiles, tiles_per_xcd;
 };
 
-// Ring cell r (0..NRING-1) -> P-plane coordinates (pi, pj): north row, south
-// row, west column, east column, corners excluded.
-__device__ __forceinline__ int2 ring_cell(int r) {
-    const bool ns = r < 2 * BX;                       // north / south rows
-    const int rr = ns ? r : r - 2 * BX;               // else west / east columns
-    const int pi = ns ? 1 + (rr % BX) : (rr < BY ? 0 : PX - 1);
-    const int pj = ns ? (rr < BX ? 0 : PY - 1) : 1 + (rr % BY);
-    return make_int2(pi, pj);
-}
-
-// Static metrics of a predicted cell: tarea_r, the four face products
-// htw*hun (i+1, i), hts*hue (j, j-1) and the del2 stencil (DTN..DTW, AHF).
-struct Metrics {
-    double tr, D1, D2, D3, D4, dtn, dts, dte, dtw, ahf;
-};
-
-__device__ __forceinline__ Metrics load_metrics(const KGrid &g, int gj, int gi) {
-    const size_t q = (size_t)gj * g.imt + gi, sj = g.imt;
-    Metrics m;
-    m.tr = g.tarea_r[q];
-    m.D1 = g.htw[q + 1] * g.hun[q + 1];
-    m.D2 = g.htw[q] * g.hun[q];
-    m.D3 = g.hts[q] * g.hue[q];
-    m.D4 = g.hts[q - sj] * g.hue[q - sj];
-    m.dtn = g.dtn[q];
-    m.dts = g.dts[q];
-    m.dte = g.dte[q];
-    m.dtw = g.dtw[q];
-    m.ahf = g.ahf[q];
-    return m;
-}
-
-// LW terms carried from the predictor of level k to the limiter of level k.
-struct LW {
-    double xy1, xy2, xy3, xy4, zb1, zb2;
-};
-
-// Staged planes of the levels around the one being predicted.
-struct Lv {
-    const double *Pk, *Pu, *Pd;     // at of levels K, K-1, K+1
-    const double *U, *V, *Wk, *Wb;  // u_wface, v_sface of level K; ws at K and K+1
-};
-
-// Predictor and limiter flag of level K at R-plane index r.
-__device__ __forceinline__ bool pred_flag(const KGrid &g, int r, const Lv &L, const int *sK, int K,
-                                          const double *odzp, const double *odzt, double dts,
-                                          double tr, double D1, double D2, double D3, double D4,
-                                          LW &lw) {
-    const double Tc = L.Pk[r], Te = L.Pk[r + 1], Tw = L.Pk[r - 1], Ts = L.Pk[r + RX],
-                 Tn = L.Pk[r - RX];
-    const double Tu = K > 0 ? L.Pu[r] : 0.0;
-    const double Td = K < g.km - 1 ? L.Pd[r] : 0.0;
-    const double Ue = L.U[r + 1], Uw = L.U[r], Vs = L.V[r], Vn = L.V[r - RX];
-    const double Wk = L.Wk[r], Wb = K < g.km - 1 ? L.Wb[r] : 0.0;
-    dev::PTerms t;
-    dev::pterms(Tc, Te, Tw, Ts, Tn, Tu, Td, Ue, Uw, Vs, Vn, Wk, Wb, tr, D1, D2, D3, D4, K, g.km,
-                odzp, odzt, dts, t);
-    lw.xy1 = t.xy1;
-    lw.xy2 = t.xy2;
-    lw.xy3 = t.xy3;
-    lw.xy4 = t.xy4;
-    lw.zb1 = t.zb1;
-    lw.zb2 = t.zb2;
-    const double a00 = dev::predictor(t, Tc, dts);
-    // 7-point bounds with land masked to -+1e10 (tracer.cpp:416-545)
-    const double lo = -1.0e10, hi = 1.0e10;
-    double mx = sK[r] > K ? Tc : lo, mn = sK[r] > K ? Tc : hi;
-    const int nb[4] = {r - RX, r + RX, r - 1, r + 1};
-    const double tv[4] = {Tn, Ts, Tw, Te};
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-        const bool wet = sK[nb[m]] > K;
-        mx = fmax(mx, wet ? tv[m] : lo);
-        mn = fmin(mn, wet ? tv[m] : hi);
-    }
-    if (K > 0) {
-        const bool wet = sK[r] > K - 1;
-        mx = fmax(mx, wet ? Tu : lo);
-        mn = fmin(mn, wet ? Tu : hi);
-    }
-    if (K < g.km - 1) {
-        const bool wet = sK[r] > K + 1;
-        mx = fmax(mx, wet ? Td : lo);
-        mn = fmin(mn, wet ? Td : hi);
-    }
-    return a00 > mx || a00 < mn;
-}
-
-// del4 first pass d2tk = AHF * del2(atb) at R-plane index r (tracer.cpp:1249-1286).
-__device__ __forceinline__ double d2tk_at(int r, const double *B, const int *sK, int k, double dtn,
-                                          double dts, double dte, double dtw, double ahf) {
-    double hdtk = 0.0, cc = 0.0;
-    if (k <= sK[r] - 1) {
-        double cf;
-        if (k <= sK[r - RX] - 1) { cf = dtn; hdtk += cf * B[r - RX]; cc -= cf; }
-        if (k <= sK[r + RX] - 1) { cf = dts; hdtk += cf * B[r + RX]; cc -= cf; }
-        if (k <= sK[r + 1] - 1) { cf = dte; hdtk += cf * B[r + 1]; cc -= cf; }
-        if (k <= sK[r - 1] - 1) { cf = dtw; hdtk += cf * B[r - 1]; cc -= cf; }
-    }
-    return ahf * (cc * B[r] + hdtk);
-}
-
-#define LDS_PTR(p) ((__attribute__((address_space(3))) void *)(p))
-
-// Direct global->LDS loads issued through inline assembly: the compiler
-// then neither reorders them nor inserts vector-memory waits before this
-// wave's later LDS reads (which touch other slots); the staging wave waits
-// for them itself (wait_vmem) before the barrier that publishes the planes.
-// M0 holds the wave's LDS destination; nothing else in these kernels uses M0.
-__device__ __forceinline__ uint32_t lds_addr(const void *p) {
-    return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)LDS_PTR(p));
-}
-__device__ __forceinline__ void dma16(const void *g, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(g)
-                 : "memory");
-}
-
-// One wave copies the R-window (tile plus 2-cell halo) of one plane straight
-// from global memory into LDS (global_load_lds: lane l of an instruction
-// lands at LDS base + 16 l), in 16-byte chunks, which needs an even imt and
-// 16-byte aligned arrays (the launcher checks).  off[u] is this lane's chunk
-// offset for instruction u inside the plane, clamped into the plane, so
-// window cells outside the array receive other cells' values, which only
-// feed cells whose results are discarded.  The loads complete asynchronously
-// (vmcnt).
-constexpr int NCH = NR / 2;                 // 16-byte chunks per window
-constexpr int NCI = (NCH + 63) / 64;        // instructions per window
-__device__ __forceinline__ void stage_plane(const double *src, double *dst, const int (&off)[NCI],
-                                            int lane) {
-#pragma unroll
-    for (int u = 0; u < NCI; ++u)
-        if (u * 64 + lane < NCH)
-            dma16(src + off[u], lds_addr(dst + 128 * u));
-}
-
-// The 16x12 tile of one plane (akt: read only at the tile's own cells):
-// 12 rows of 16 doubles, 8 chunks per row, 96 chunks in two instructions;
-// chunk c lands at element 2c of the slot, which is the tile lane index.
-constexpr int NCA = BX * BY / 2;
-__device__ __forceinline__ void stage_tile(const double *src, double *dst, const int (&off)[2],
-                                           int lane) {
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-        if (u * 64 + lane < NCA)
-            dma16(src + off[u], lds_addr(dst + 128 * u));
-}
-
-__device__ __forceinline__ void wait_vmem() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-// Waits for every staged load except the `issued` issued at the start of
-// the current level (direct-to-LDS loads complete in order).
-__device__ __forceinline__ void wait_vmem_keep(int issued) {
-    static_assert(DMA_ATW + DMA_UVBA == 17 && DMA_UVBA == 11, "wait counts below");
-    if (LA < 2 || issued == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    else if (issued >= 17) asm volatile("s_waitcnt vmcnt(17)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(11)" ::: "memory");
-}
-
-// Workgroup barrier that waits only for this wave's LDS traffic.  The
-// staging wave's direct-to-LDS loads are waited for explicitly (wait_vmem)
-// before the barrier that publishes them, so the tile waves never wait on
-// vector-memory counters at a barrier.
-__device__ __forceinline__ void bar_lds() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-// k-march over one 16x12 tile of columns and one tracer, four waves.
-// Waves 0-2 own the tile's cells; wave 3 owns the 56 ring cells the limiter
-// and the del4 second pass read around the tile, and stages every plane
-// (a four-wave workgroup keeps three workgroups resident per CU).
-// Per level k two phases, each closed by a barrier:
-//   P(k): wave 3 first issues the direct-to-LDS loads of the planes first
-//         read LA levels later; then the tspas predictor of level k+1 and
-//         the del4 first pass of level k at every cell (tile and ring, one
-//         cell per lane).
-//   C(k): limiter, fluxes and explicit update of level k on the tile (waves
-//         0-2); wave 3 waits for the loads P(k+1) and C(k+1) read.
-// LDS slots rotate: at and ws x(LA+3), u_wface/v_sface, atb and akt x(LA+2).
-// ADV: the advection scheme (LICOM_ADV_*); centered and flux need no
-// predictor, so their P(k) is the del4 first pass alone.
-template <int ADV>
-__global__ __launch_bounds__(NT, (LA >= 2 ? 2 : 3)) void k_march(KGrid g, KPar p, MarchArgs a) {
+// Limited fluxes, horizontal mixing, shortwave and explicit vertical
+// diffusion of every interior cell: tracer_8's explicit update (ori) and the
+// ax/ay/az/dz/penetrate diagnostics.  The biharmonic operator's first pass is
+// formed again for the rows on both sides of the lane's own (two more loads
+// of atb a level, where its 16 bytes a cell would be written and read back).
+template <int ADV, bool DEL4>
+__global__ __launch_bounds__(256, DEL4 ? 2 : 3) void k_update(KGrid g, KPar p, const double *__restrict__ at,
+                                                   const double *__restrict__ atb, const double *__restrict__ akt,
+                                                   const double *__restrict__ uw, const double *__restrict__ vs,
+                                                   const double *__restrict__ ws, const uint8_t *__restrict__ flags,
+                                                   double *__restrict__ ori, const double *__restrict__ odzp,
+                                                   const double *__restrict__ odzt, const double *__restrict__ penk,
+                                                   UpdateArgs a, FlatGrid fg) {
     constexpr bool tspas = ADV == LICOM_ADV_TSPAS;
-    __shared__ __align__(16) double sAT[NAT][NR];
-    __shared__ __align__(16) double sU[NUV][NR];
-    __shared__ __align__(16) double sV[NUV][NR];
-    __shared__ __align__(16) double sW[NW][NR];
-    __shared__ __align__(16) double sB[NB][NR];
-    __shared__ double sD2[NP];
-    __shared__ unsigned char sFL[2][NP];
-    __shared__ int sK[NR];
-    // odzp, odzt and pen: per-level constants read from LDS, so that no
-    // vector-memory load inside the level loop carries a vmcnt wait (on gfx9
-    // vmcnt also covers the staged planes, the akt prefetch and the stores)
-    __shared__ double sZP[KMAXF], sZT[KMAXF], sPN[KMAXF];
-    __shared__ __align__(16) double sAK[NB][NOWN];    // akt of the tile, staged like atb
+    int n, blk, k0;
+    if (!flat_block(fg, n, blk, k0)) return;
+    const int imt = g.imt, jmt = g.jmt, km = g.km, n2 = imt * jmt, lane = (int)threadIdx.x & 63;
+    const size_t n3 = (size_t)n2 * km;
+    const int pl = lane_cell(fg, blk);
+    const int pc = clamp_cell(pl, n2), pn = clamp_cell(pl - imt, n2), ps = clamp_cell(pl + imt, n2);
+    uint32_t bc = 8u * (uint32_t)pc, bn = 8u * (uint32_t)pn, bs = 8u * (uint32_t)ps;
+    bool own[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        const int c = pl + e, i = c % imt;
+        own[e] = lane >= 1 && lane <= 62 && c < fg.last && i >= 2 && i < imt - 2;
+    }
 
-    // XCD-aware placement: consecutive blocks of one XCD take the T and S
-    // halves of one tile, then the next tile of the same row of tiles.
-    const int Lb = blockIdx.x, xcd = Lb & 7, slot = Lb >> 3;
-    const int tile = xcd * a.tiles_per_xcd + (slot >> 1);
-    const int n = slot & 1;
-    if (tile >= a.ntiles) return;
-    const int imt = g.imt, jmt = g.jmt, km = g.km;
-    const size_t n2 = (size_t)imt * jmt, n3 = n2 * km;
-    const int gi0 = 2 + (tile % a.ntx) * BX, gj0 = 2 + (tile / a.ntx) * BY;
-    const long e0 = (long)(gj0 - 2) * imt + (gi0 - 2);
-
-    const int t = threadIdx.x, lane = t & 63;
-    // wave 3 (lanes NOWN..NT-1) is the ring/staging wave; the test goes
-    // through a scalar register so that the two roles compile to two
-    // separate loops behind a uniform branch (with a per-lane test they are
-    // merged into one exec-masked loop, and the tile waves' loads and stores
-    // then carry vmcnt waits into the staging wave's code)
-    const bool ringw = __builtin_amdgcn_readfirstlane(t >> 6) == NOWN / 64;
-    const int rl = t - NOWN;                     // ring lane (wave 3)
-    const bool has_cell = !ringw || rl < NRING;
-    const int2 rc = ring_cell(has_cell && ringw ? rl : 0);
-    const int pi = ringw ? rc.x : 1 + t % BX, pj = ringw ? rc.y : 1 + t / BX;
-    const int gi = gi0 - 1 + pi, gj = gj0 - 1 + pj;
-    const int rC = (pj + 1) * RX + (pi + 1), pC = pj * PX + pi;
-    const bool cell_ok = has_cell && gj >= 1 && gj < jmt - 1 && gi >= 1 && gi < imt - 1;
-    const bool act = !ringw && gi < imt - 2 && gj < jmt - 2;
-    const size_t q = cell_ok ? (size_t)gj * imt + gi : 0;
-
-    const double *T = a.at + n * n3;
-    const double *TB = a.atb + n * (n3 + n2) + n2;   // level k at plane k
-    const double *A = a.akt + n * n3;
+    const double *T = at + n * n3;
+    const double *TB = atb + n * (n3 + n2) + n2;     // level k at plane k
+    const double *A = akt + n * n3;
+    const uint8_t *F = flags + n * n3;
     const double dts = p.dts;
-
-    for (int r = t; r < NR; r += NT) {
-        const int rj = gj0 - 2 + r / RX, ri = gi0 - 2 + r % RX;
-        sK[r] = (rj < jmt && ri < imt) ? g.kmt[(size_t)rj * imt + ri] : 0;
+    int kmt[2];
+    double sw[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        kmt[e] = g.kmt[pc + e];
+        sw[e] = (n == 0 && a.swv) ? a.swv[pc + e] : 0.0;
     }
-    for (int r = t; r < km; r += NT) {
-        sZP[r] = g.odzp[r];
-        sZT[r] = g.odzt[r];
-        sPN[r] = r < km - 1 ? g.pen[r] : 0.0;
-    }
-    Metrics M{};
-    if (cell_ok) M = load_metrics(g, gj, gi);
-    const double sw = (n == 0 && act && a.swv) ? a.swv[q] : 0.0;
-    const int kmt_own = act ? g.kmt[q] : 0;
-    const double stf_n = act ? a.stf_n[n * n2 + q] : 0.0;
-    const double enorm = (n == 1 && p.sssnorm && act) ? a.err_norm2[0] : 0.0;
     const bool rest = p.boundary_restore == 1 && a.restore != nullptr;
-
-    if (ringw) {
-        // ---- wave 3: ring cells and plane staging
-        int off[NCI];
-#pragma unroll
-        for (int u = 0; u < NCI; ++u) {
-            const int c = min(u * 64 + lane, NCH - 1), row = c / (RX / 2), cp = c - row * (RX / 2);
-            off[u] = (int)min(e0 + (long)row * imt + 2 * cp, (long)n2 - 2);
-        }
-        int offa[2];
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int c = min(u * 64 + lane, NCA - 1), row = c / (BX / 2), cp = c - row * (BX / 2);
-            offa[u] = (int)min((long)(gj0 + row) * imt + gi0 + 2 * cp, (long)n2 - 2);
-        }
-        // prologue: at, ws 0..LA+1; faces, atb, akt 0..LA
-        for (int l = 0; l < NAT - 1 && l < km; ++l) {
-            stage_plane(T + (size_t)l * n2, sAT[l], off, lane);
-            stage_plane(a.ws + (size_t)l * n2, sW[l], off, lane);
-        }
-        for (int l = 0; l < NUV - 1 && l < km; ++l) {
-            stage_plane(a.uw + (size_t)l * n2, sU[l], off, lane);
-            stage_plane(a.vs + (size_t)l * n2, sV[l], off, lane);
-            stage_plane(TB + (size_t)l * n2, sB[l], off, lane);
-            stage_tile(A + (size_t)l * n2, sAK[l], offa, lane);
-        }
-        wait_vmem();
-        bar_lds();
-        if constexpr (tspas) {
-            LW tmp;
-            const Lv L0{sAT[0], sAT[0], sAT[1], sU[0], sV[0], sW[0], sW[1]};
-            const bool f0 = cell_ok ? pred_flag(g, rC, L0, sK, 0, sZP, sZT, dts, M.tr, M.D1, M.D2, M.D3,
-                                                M.D4, tmp)
-                                    : false;
-            if (has_cell) sFL[0][pC] = f0;
-        }
-        bar_lds();
-        for (int k = 0; k < km; ++k) {
-            const int s0 = k % NAT, s1 = (k + 1) % NAT, s2 = (k + 2) % NAT, s3 = (k + LA + 2) % NAT;
-            const int u0 = k % NUV, u1 = (k + 1) % NUV, u2 = (k + LA + 1) % NUV;
-            // planes for P(k+LA) and C(k+LA), issued first so that they have
-            // LA levels to land; their slots were last read in C(k-1)
-            int issued = 0;
-            if (k + LA + 2 < km) {
-                stage_plane(T + (size_t)(k + LA + 2) * n2, sAT[s3], off, lane);
-                stage_plane(a.ws + (size_t)(k + LA + 2) * n2, sW[s3], off, lane);
-                issued += DMA_ATW;
-            }
-            if (k + LA + 1 < km) {
-                stage_plane(a.uw + (size_t)(k + LA + 1) * n2, sU[u2], off, lane);
-                stage_plane(a.vs + (size_t)(k + LA + 1) * n2, sV[u2], off, lane);
-                stage_plane(TB + (size_t)(k + LA + 1) * n2, sB[u2], off, lane);
-                stage_tile(A + (size_t)(k + LA + 1) * n2, sAK[u2], offa, lane);
-                issued += DMA_UVBA;
-            }
-            if (tspas && k + 1 < km) {
-                LW tmp;
-                const Lv L1{sAT[s1], sAT[s0], sAT[s2], sU[u1], sV[u1], sW[s1], sW[s2]};
-                const bool f =
-                    cell_ok ? pred_flag(g, rC, L1, sK, k + 1, sZP, sZT, dts, M.tr, M.D1, M.D2, M.D3,
-                                        M.D4, tmp)
-                            : false;
-                if (has_cell) sFL[(k + 1) & 1][pC] = f;
-            }
-            if (p.hmix == LICOM_HMIX_DEL4 && has_cell)
-                sD2[pC] = cell_ok ? d2tk_at(rC, sB[u0], sK, k, M.dtn, M.dts, M.dte, M.dtw, M.ahf) : 0.0;
-            bar_lds();                // end of P(k)
-            wait_vmem_keep(issued);   // C(k): the planes P(k+1) and C(k+1) read land
-            bar_lds();                // end of C(k)
-        }
-        return;
-    }
-
-    // ---- waves 0-2: the tile
-    // the per-cell loads above complete here, before the level loop, so
-    // that no wait for them (which would also wait for the level's stores)
-    // stays inside it
-    __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
-    bar_lds();
-    LW lc{}, ln{};
-    if constexpr (tspas) {
-        const Lv L0{sAT[0], sAT[0], sAT[1], sU[0], sV[0], sW[0], sW[1]};
-        sFL[0][pC] = cell_ok ? pred_flag(g, rC, L0, sK, 0, sZP, sZT, dts, M.tr, M.D1, M.D2, M.D3, M.D4,
-                                         lc)
-                             : false;
-    }
-    bar_lds();
-
-    double Tprev = 0.0, Bprev = 0.0, Aprev = 0.0;
-    bool fprev = false;
     const double lamda = 1.0 / (15.0 * 86400.0);
     const double aidif = 0.5;
 
-    for (int k = 0; k < km; ++k) {
-        const int s0 = k % NAT, s1 = (k + 1) % NAT, s2 = (k + 2) % NAT;
-        const int u0 = k % NUV, u1 = (k + 1) % NUV;
-        // ---- phase P(k)
-        const double Acur = act ? dev::floor_akt(sAK[u0][t], k, n, p.hmix, p.dwndmix) : 0.0;
-        if (tspas && k + 1 < km) {
-            const Lv L1{sAT[s1], sAT[s0], sAT[s2], sU[u1], sV[u1], sW[s1], sW[s2]};
-            sFL[(k + 1) & 1][pC] =
-                cell_ok ? pred_flag(g, rC, L1, sK, k + 1, sZP, sZT, dts, M.tr, M.D1, M.D2, M.D3, M.D4,
-                                    ln)
-                        : false;
-        }
-        if (p.hmix == LICOM_HMIX_DEL4)
-            sD2[pC] = cell_ok ? d2tk_at(rC, sB[u0], sK, k, M.dtn, M.dts, M.dte, M.dtw, M.ahf) : 0.0;
-        bar_lds();
+    // The lane's metrics wait in LDS and are read anew at each level: in
+    // registers they would leave too few for the level's loads and waves.
+    // del4 adds the stencils of the rows on both sides (outer rows bN, bS).
+    __shared__ licom_d2a sM[DEL4 ? 19 : 8][256];
+    auto keep = [&](int slot, double x, double y) { sM[slot][threadIdx.x] = licom_d2a{x, y}; };
+    auto get = [&](int slot) {
+        const licom_d2a x = sM[slot][threadIdx.x];
+        return D2{{x.x, x.y}};
+    };
+    {
+        const Faces fc = load_faces(g, pc, pn);
+        keep(0, fc.tr[0], fc.tr[1]);
+        keep(1, fc.dx[0], fc.dx[1]);
+        keep(2, fc.ds[0], fc.ds[1]);
+        keep(3, fc.dn[0], fc.dn[1]);
+    }
+    uint32_t wet[3][2];
+    uint32_t bN = 0, bS = 0;
+    load_wet(g, pc, pn, ps, wet[0]);
+    if constexpr (DEL4) {
+        const int pN = clamp_cell(pl - 2 * imt, n2), pS = clamp_cell(pl + 2 * imt, n2);
+        load_wet(g, pn, pN, pc, wet[1]);
+        load_wet(g, ps, pc, pS, wet[2]);
+        bN = 8u * (uint32_t)pN;
+        bS = 8u * (uint32_t)pS;
+    }
+    {
+        const double *co[5] = {g.dtn, g.dts, g.dte, g.dtw, g.ahf};
+#pragma unroll
+        for (int r = 0; r < (DEL4 ? 3 : 1); ++r)
+#pragma unroll
+            for (int c = 0; c < (DEL4 ? 5 : 4); ++c) {
+                const int cell = r == 0 ? pc : (r == 1 ? pn : ps);
+                keep(4 + r * 5 + c, co[c][cell], co[c][cell + 1]);
+            }
+    }
+    auto stencil = [&](int r) { return Del2{get(4 + r * 5), get(5 + r * 5), get(6 + r * 5), get(7 + r * 5)}; };
 
-        // ---- phase C(k): limited fluxes and the explicit update of level k
-        if (act) {
-            const double *Pk = sAT[s0], *Pk1 = sAT[s1];
-            const double *Bk = sB[u0], *Bk1 = sB[u1];
-            const unsigned char *F = sFL[k & 1];
-            const int r = rC, pp = pC;
-            const double Tc = Pk[r], Te = Pk[r + 1], Tw = Pk[r - 1], Ts = Pk[r + RX], Tn = Pk[r - RX];
-            const double Tu = Tprev, Td = (k + 1 < km) ? Pk1[r] : 0.0;
-            const double *U = sU[u0], *V = sV[u0];
-            const double Ue = U[r + 1], Uw = U[r], Vs = V[r], Vn = V[r - RX];
-            const double Wk = sW[s0][r], Wb = (k + 1 < km) ? sW[s1][r] : 0.0;
-            const size_t c = (size_t)k * n2 + q;
-            const double vk = k < kmt_own ? 1.0 : 0.0;
+    const int k1 = min(k0 + fg.kc, km);
+    const size_t o0 = (size_t)k0 * n2;
+    D2 Tu{}, Bu{}, Au{}, Tc = ld2(T + o0, bc), Bc = ld2(TB + o0, bc), Wk = ld2(ws + o0, bc);
+    uint32_t fu = 0, f0 = 0;
+    if constexpr (tspas) f0 = ldf2(F + o0, (uint32_t)pc);
+    if (k0 > 0) {
+        Tu = ld2(T + o0 - n2, bc);
+        Bu = ld2(TB + o0 - n2, bc);
+        Au = ld2(A + o0 - n2, bc);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) Au.v[e] = dev::floor_akt(Au.v[e], k0 - 1, n, p.hmix, p.dwndmix);
+        if constexpr (tspas) fu = ldf2(F + o0 - n2, (uint32_t)pc);
+    }
+
+    march_levels(k0, k1, km, [&](auto pos, int k) {
+        constexpr bool top = pos == 0, bot = pos == 2;
+        // the shared expressions tell first, inner and last levels apart
+        constexpr int kp = top ? 0 : 1, kq = bot ? 2 : 3;
+        const double oz = odzp[k], ot = odzt[k], ot1 = bot ? 0.0 : odzt[k + 1];
+        const double pe = bot ? 0.0 : penk[k], peu = top ? 0.0 : penk[k - 1];
+        const size_t o = (size_t)k * n2, on = n * n3 + o;
+        fresh(bc);
+        fresh(bn);
+        fresh(bs);
+        if constexpr (DEL4) {
+            fresh(bN);
+            fresh(bS);
+        }
+        const D2 Tn = ld2(T + o, bn), Ts = ld2(T + o, bs);
+        const D2 Bn = ld2(TB + o, bn), Bs = ld2(TB + o, bs);
+        const D2 U = ld2(uw + o, bc), Vs = ld2(vs + o, bc), Vn = ld2(vs + o, bn);
+        D2 Ac = ld2(A + o, bc), Td{}, Wb{}, Bd{}, BN{}, BS{}, Rk{};
+        uint32_t fd = 0, fn = 0, fs = 0;
+        if constexpr (DEL4) {
+            BN = ld2(TB + o, bN);
+            BS = ld2(TB + o, bS);
+        }
+        if constexpr (tspas) {
+            fn = ldf2(F + o, bn >> 3);
+            fs = ldf2(F + o, bs >> 3);
+        }
+        if constexpr (!bot) {
+            Td = ld2(T + o + n2, bc);
+            Bd = ld2(TB + o + n2, bc);
+            Wb = ld2(ws + o + n2, bc);
+            if constexpr (tspas) fd = ldf2(F + o + n2, bc >> 3);
+        }
+        const bool rk = !top && rest;
+        if (rk) Rk = ld2(a.restore + on, bc);
+        const D2 Tw = west(Tc), Te = east(Tc), Bw = west(Bc), Be = east(Bc), Ue = east(U);
+        // horizontal mixing (tracer_del4_2 / tracer_4)
+        double hm[2];
+        asm volatile("" ::: "memory");
+        const Del2 M = stencil(0);
+        if constexpr (DEL4) {
+            const D2 Nw = west(Bn), Ne = east(Bn), Sw = west(Bs), Se = east(Bs);
+            D2 dc, dn, ds;
+            {
+                const Del2 R = stencil(1);
+                const D2 ahf = get(13);
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+                    dn.v[e] = ahf.v[e] * del2(R, wet[1][e], e, k, Bn.v[e], BN.v[e], Bc.v[e], Ne.v[e], Nw.v[e]);
+            }
+            {
+                const Del2 R = stencil(2);
+                const D2 ahf = get(18);
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+                    ds.v[e] = ahf.v[e] * del2(R, wet[2][e], e, k, Bs.v[e], Bc.v[e], BS.v[e], Se.v[e], Sw.v[e]);
+            }
+            const D2 ahf = get(8);
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+                dc.v[e] = ahf.v[e] * del2(M, wet[0][e], e, k, Bc.v[e], Bn.v[e], Bs.v[e], Be.v[e], Bw.v[e]);
+            const D2 dw = west(dc), de = east(dc);
+#pragma unroll
+            for (int e = 0; e < 2; ++e) hm[e] = del2(M, wet[0][e], e, k, dc.v[e], dn.v[e], ds.v[e], de.v[e], dw.v[e]);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 2; ++e) hm[e] = del2(M, wet[0][e], e, k, Bc.v[e], Bn.v[e], Bs.v[e], Be.v[e], Bw.v[e]);
+        }
+        // limiter flags of the cells to the west and east
+        const uint32_t fw = ((uint32_t)dpp<kFromPrev>((int)f0) >> 8) | (f0 << 8);
+        const uint32_t fe = (f0 >> 8) | ((uint32_t)dpp<kFromNext>((int)f0) << 8);
+        const D2 mtr = get(0), mdx = get(1), mds = get(2), mdn = get(3);
+        const double mde[2] = {mdx.v[1], dppd<kFromNext>(mdx.v[0])};
+        double xx[2], yy[2], zz[2], dzv[2], pv[2], out[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const double tc = Tc.v[e], wk = Wk.v[e], wb = Wb.v[e], tr = mtr.v[e];
+            const double vk = k < kmt[e] ? 1.0 : 0.0;
             double tf;
-            bool fc = false;
             if constexpr (!tspas) {
                 // advection_tracer_1 (tracer.cpp:120-289); the centered form
                 // accumulates its diagnostics (the caller's ax/ay/az carry the
                 // sum over the diagnostic period)
-                const dev::CFAdv cf = dev::adv_cf(ADV, Tc, Te, Tw, Ts, Tn, Tu, Td, Ue, Uw, Vs, Vn, Wk, Wb, M.tr,
-                                                  k, km, sZP);
-                if constexpr (ADV == LICOM_ADV_CENTERED) {
-                    const double nss = (double)p.nss;
-                    if (a.ax) a.ax[n * n3 + c] = a.ax[n * n3 + c] + cf.hx / nss;
-                    if (a.ay) a.ay[n * n3 + c] = a.ay[n * n3 + c] + cf.hy / nss;
-                    if (a.az) a.az[n * n3 + c] = a.az[n * n3 + c] - cf.vz / nss;
-                }
+                const dev::CFAdv cf = dev::adv_cf(ADV, tc, Te.v[e], Tw.v[e], Ts.v[e], Tn.v[e], Tu.v[e], Td.v[e],
+                                                  Ue.v[e], U.v[e], Vs.v[e], Vn.v[e], wk, wb, tr, kp, kq, oz);
+                const double nss = (double)p.nss;
+                xx[e] = cf.hx / nss;
+                yy[e] = cf.hy / nss;
+                zz[e] = cf.vz / nss;
                 tf = cf.adv * vk;
             } else {
-                fc = F[pp];
-                const bool fe = F[pp + 1], fw = F[pp - 1], fs = F[pp + PX], fn = F[pp - PX];
-                const bool fd = (k + 1 < km) ? sFL[(k + 1) & 1][pp] : false;
-                bool up1, up2, up3, up4;
-                if (k == 0 || k == km - 1) {
-                    up1 = fc || (fe && gi <= imt - 3);
-                    up2 = fc || (fw && gi >= 2);
-                    up3 = fc || (fs && gj <= jmt - 3);
-                    up4 = fc || (fn && gj >= 2);
-                } else {
-                    up1 = (fc || fe) && gi <= imt - 3;
-                    up2 = (fc || fw) && gi >= 2;
-                    up3 = (fc || fs) && gj <= jmt - 3;
-                    up4 = (fc || fn) && gj >= 2;
-                }
-                const double tr = M.tr;
-                dev::PTerms tc;
-                dev::pterms_cheap(Tc, Te, Tw, Ts, Tn, Tu, Td, Ue, Uw, Vs, Vn, Wk, Wb, tr, k, km, sZP, tc);
-                const double xy1 = up1 ? dev::up_xy1(Te, Tc, Ue, tr) : lc.xy1;
-                const double xy2 = up2 ? dev::up_xy2(Tc, Tw, Uw, tr) : lc.xy2;
-                const double xy3 = up3 ? dev::up_xy1(Ts, Tc, Vs, tr) : lc.xy3;
-                const double xy4 = up4 ? dev::up_xy2(Tc, Tn, Vn, tr) : lc.xy4;
-                double zb1, zb2;
-                if (k == 0) {
-                    zb1 = 0.0;
-                    zb2 = (fc || fd) ? dev::up_zb2(Tc, Td, Wb, sZP[0]) : lc.zb2;
-                } else if (k == km - 1) {
-                    zb1 = (fc || fprev) ? dev::up_zb1(Tu, Tc, Wk, sZP[k]) : lc.zb1;
-                    zb2 = 0.0;
-                } else {
-                    zb1 = (fc || fprev) ? dev::up_zb1(Tu, Tc, Wk, sZP[k]) : lc.zb1;
-                    zb2 = (fc || fd) ? dev::up_zb2(Tc, Td, Wb, sZP[k]) : lc.zb2;
-                }
-                const double xx = -(tc.x0 + xy1 + xy2 + tc.c1);
-                const double yy = -(tc.y0 + xy3 + xy4 + tc.c2);
-                const double zz = -(tc.za + zb1 + zb2 + tc.zc);
-                if (a.ax) a.ax[n * n3 + c] = xx;
-                if (a.ay) a.ay[n * n3 + c] = yy;
-                if (a.az) a.az[n * n3 + c] = zz;
-                tf = (xx + yy + zz) * vk;
+                const bool lim = (f0 >> (8 * e)) & 1u;
+                dev::PTerms t;
+                dev::pterms(tc, Te.v[e], Tw.v[e], Ts.v[e], Tn.v[e], Tu.v[e], Td.v[e], Ue.v[e], U.v[e], Vs.v[e],
+                            Vn.v[e], wk, wb, tr, mde[e], mdx.v[e], mds.v[e], mdn.v[e], kp, kq, oz, ot, ot1, dts, t);
+                // a face is upwind where a cell beside it is limited
+                // (tracer.cpp:574-658; every face of an interior cell passes
+                // the reference's index tests)
+                auto up = [&](uint32_t f) { return lim || ((f >> (8 * e)) & 1u); };
+                const double xy1 = up(fe) ? dev::up_xy1(Te.v[e], tc, Ue.v[e], tr) : t.xy1;
+                const double xy2 = up(fw) ? dev::up_xy2(tc, Tw.v[e], U.v[e], tr) : t.xy2;
+                const double xy3 = up(fs) ? dev::up_xy1(Ts.v[e], tc, Vs.v[e], tr) : t.xy3;
+                const double xy4 = up(fn) ? dev::up_xy2(tc, Tn.v[e], Vn.v[e], tr) : t.xy4;
+                double zb1 = 0.0, zb2 = 0.0;
+                if constexpr (!top) zb1 = up(fu) ? dev::up_zb1(Tu.v[e], tc, wk, oz) : t.zb1;
+                if constexpr (!bot) zb2 = up(fd) ? dev::up_zb2(tc, Td.v[e], wb, oz) : t.zb2;
+                xx[e] = -(t.x0 + xy1 + xy2 + t.c1);
+                yy[e] = -(t.y0 + xy3 + xy4 + t.c2);
+                zz[e] = -(t.za + zb1 + zb2 + t.zc);
+                tf = (xx[e] + yy[e] + zz[e]) * vk;
             }
-            // horizontal mixing (tracer_del4_2 / tracer_4)
-            {
-                const bool d4 = p.hmix == LICOM_HMIX_DEL4;
-                const double *X = d4 ? sD2 : Bk;
-                const int xs = d4 ? pp : r, xw = d4 ? PX : RX;
-                double hdtk = 0.0, cc = 0.0;
-                if (k <= sK[r] - 1) {
-                    double cf;
-                    if (k <= sK[r - RX] - 1) { cf = M.dtn; hdtk += cf * X[xs - xw]; cc -= cf; }
-                    if (k <= sK[r + RX] - 1) { cf = M.dts; hdtk += cf * X[xs + xw]; cc -= cf; }
-                    if (k <= sK[r + 1] - 1) { cf = M.dte; hdtk += cf * X[xs + 1]; cc -= cf; }
-                    if (k <= sK[r - 1] - 1) { cf = M.dtw; hdtk += cf * X[xs - 1]; cc -= cf; }
-                }
-                tf += p.ah * (cc * X[xs] + hdtk);
-            }
+            tf += p.ah * hm[e];
             // shortwave penetration (T) and explicit vertical diffusion
             // (tracer_5, boundary levels as its k==0 thread applies them)
-            const double *odzp = sZP, *odzt = sZT;
-            const double v1 = (k + 1 < km && k + 1 < kmt_own) ? 1.0 : 0.0;
-            if (n == 0) {
-                double pv;
-                if (k == 0) {
-                    const double wt1 = sw * sPN[0] * (1 < kmt_own ? 1.0 : 0.0);
-                    tf = tf - odzp[0] * wt1;
-                    pv = -wt1 * odzp[0];
-                } else if (k == km - 1) {
-                    const double wt2 = sw * sPN[km - 2] * vk;
-                    tf = tf + odzp[km - 1] * wt2;
-                    pv = wt2 * odzp[km - 1];
+            const double v1 = (!bot && k + 1 < kmt[e]) ? 1.0 : 0.0;
+            {
+                double ts;
+                if constexpr (top) {
+                    const double wt1 = sw[e] * pe * (1 < kmt[e] ? 1.0 : 0.0);
+                    ts = tf - oz * wt1;
+                    pv[e] = -wt1 * oz;
+                } else if constexpr (bot) {
+                    const double wt2 = sw[e] * peu * vk;
+                    ts = tf + oz * wt2;
+                    pv[e] = wt2 * oz;
                 } else {
-                    const double wt1 = sw * sPN[k - 1] * vk;
-                    const double wt2 = sw * sPN[k] * v1;
-                    tf = tf + (wt1 - wt2) * odzp[k];
-                    pv = (wt1 - wt2) * odzp[k];
+                    const double wt1 = sw[e] * peu * vk;
+                    const double wt2 = sw[e] * pe * v1;
+                    ts = tf + (wt1 - wt2) * oz;
+                    pv[e] = (wt1 - wt2) * oz;
                 }
-                if (a.pen) a.pen[c] = pv;
+                tf = n == 0 ? ts : tf;
             }
-            const double Bc = Bk[r];
-            double dzv;
-            if (k == 0) {
-                const double wt1 = Acur * (Bc - Bk1[r]) * odzt[1] * v1;
-                tf = tf - odzp[0] * wt1 * 0.5;
-                dzv = -odzp[0] * wt1 * 0.5;
-            } else if (k == km - 1) {
-                const double wt2 = Aprev * (Bprev - Bc) * odzt[km - 1] * vk;
-                tf = tf + odzp[km - 1] * wt2 * (1.0 - aidif);
-                dzv = odzp[km - 1] * wt2 * 0.5;
+            Ac.v[e] = dev::floor_akt(Ac.v[e], k, n, p.hmix, p.dwndmix);
+            const double b = Bc.v[e];
+            if constexpr (top) {
+                const double wt1 = Ac.v[e] * (b - Bd.v[e]) * ot1 * v1;
+                tf = tf - oz * wt1 * 0.5;
+                dzv[e] = -oz * wt1 * 0.5;
+            } else if constexpr (bot) {
+                const double wt2 = Au.v[e] * (Bu.v[e] - b) * ot * vk;
+                tf = tf + oz * wt2 * (1.0 - aidif);
+                dzv[e] = oz * wt2 * 0.5;
             } else {
-                const double wt1 = Aprev * (Bprev - Bc) * odzt[k] * vk;
-                const double wt2 = Acur * (Bc - Bk1[r]) * odzt[k + 1] * v1;
-                tf = tf + odzp[k] * (wt1 - wt2) * 0.5;
-                dzv = odzp[k] * (wt1 - wt2) * 0.5;
+                const double wt1 = Au.v[e] * (Bu.v[e] - b) * ot * vk;
+                const double wt2 = Ac.v[e] * (b - Bd.v[e]) * ot1 * v1;
+                tf = tf + oz * (wt1 - wt2) * 0.5;
+                dzv[e] = oz * (wt1 - wt2) * 0.5;
             }
-            if (a.dz) a.dz[n * n3 + c] = dzv;
-            if (a.flags_out) a.flags_out[n * n3 + c] = fc;
             // surface fluxes (tracer_5 n=1, tracer_6) and restoring (tracer_7)
-            if (k == 0) {
+            if constexpr (top) {
+                const double stf = a.stf_n[(size_t)n * n2 + pc + e];
                 if (n == 1) {
-                    if (kmt_own > 0) tf = tf + stf_n * (1.0 - aidif) * odzp[0];
-                    if (p.sssnorm) tf = tf + enorm * vk;
-                } else if (kmt_own > 0) {
-                    tf = tf + stf_n * odzp[0] * 0.5;
+                    if (kmt[e] > 0) tf = tf + stf * (1.0 - aidif) * oz;
+                    if (p.sssnorm) tf = tf + a.err_norm2[0] * vk;
+                } else if (kmt[e] > 0) {
+                    tf = tf + stf * oz * 0.5;
                 }
             }
-            if (rest && k >= 1) {
-                const double Rk = a.restore[n * n3 + c];
-                tf = tf + vk * (Rk - Bc) * lamda;
-            }
+            if (rk) tf = tf + vk * (Rk.v[e] - b) * lamda;
             // tracer_8: the explicit update entering the implicit solve
-            a.ori[n * n3 + c] = Tc + dts * tf;
-            Tprev = Tc;
-            Bprev = Bc;
-            fprev = fc;
+            out[e] = tc + dts * tf;
         }
-        Aprev = Acur;
-        lc = ln;
-        bar_lds();
+        if constexpr (ADV == LICOM_ADV_CENTERED) {
+            auto add = [&](double *d, double sign, const double (&x)[2]) {
+                const D2 y = ld2(d + on, bc);
+                const double s[2] = {y.v[0] + sign * x[0], y.v[1] + sign * x[1]};
+                st2(d + on, bc, s, own[0], own[1]);
+            };
+            if (a.ax) add(a.ax, 1.0, xx);
+            if (a.ay) add(a.ay, 1.0, yy);
+            if (a.az) add(a.az, -1.0, zz);
+        } else if constexpr (tspas) {
+            if (a.ax) st2(a.ax + on, bc, xx, own[0], own[1]);
+            if (a.ay) st2(a.ay + on, bc, yy, own[0], own[1]);
+            if (a.az) st2(a.az + on, bc, zz, own[0], own[1]);
+        }
+        if (n == 0 && a.pen) st2(a.pen + o, bc, pv, own[0], own[1]);
+        if (a.dz) st2(a.dz + on, bc, dzv, own[0], own[1]);
+        if (a.flags_out) {
+            if (own[0]) a.flags_out[on + (bc >> 3)] = (uint8_t)(f0 & 1u);
+            if (own[1]) a.flags_out[on + (bc >> 3) + 1] = (uint8_t)(f0 >> 8);
+        }
+        st2(ori + on, bc, out, own[0], own[1]);
+        Tu = Tc;
+        Tc = Td;
+        Bu = Bc;
+        Bc = Bd;
+        Au = Ac;
+        Wk = Wb;
+        fu = f0;
+        f0 = fd;
+    });
+}
+
+template <int ADV>
+void launch_update(licom_ctx *ctx, const licom_fields *f, const licom_diag *d, const Scratch &s) {
+    const KGrid &g = ctx->g;
+    hipStream_t st = ctx->stream;
+    Timer t(ctx, "k_march");     // one name for both, as in the mixed form
+    if constexpr (ADV == LICOM_ADV_TSPAS) {
+        const FlatGrid fg = flat_grid(g.imt, (g.jmt - 1) * g.imt, g.km);
+        k_flags<<<8 * fg.per, 256, 0, st>>>(g, ctx->kp.dts, f->at, s.uw, s.vs, f->ws, s.flags, g.odzp, g.odzt, fg);
     }
+    UpdateArgs a{};
+    a.stf_n = s.stf_n;
+    a.err_norm2 = s.err_norm2;
+    a.swv = f->swv;
+    a.restore = f->restore;
+    a.ax = d ? d->ax : nullptr;
+    a.ay = d ? d->ay : nullptr;
+    a.az = d ? d->az : nullptr;
+    a.dz = d ? d->dz : nullptr;
+    a.pen = d ? d->penetrate : nullptr;
+    a.flags_out = ctx->flags_out;
+    const FlatGrid fg = flat_grid(2 * g.imt, (g.jmt - 2) * g.imt, g.km);
+    auto kern = ctx->kp.hmix == LICOM_HMIX_DEL4 ? k_update<ADV, true> : k_update<ADV, false>;
+    kern<<<8 * fg.per, 256, 0, st>>>(g, ctx->kp, f->at, f->atb, f->akt, s.uw, s.vs, f->ws, s.flags, s.ori, g.odzp,
+                                     g.odzt, g.pen, a, fg);
 }
 
 // Side effects of tracer_1_0 / tracer_1 / tracer_del4_2 (tracer.cpp:1088,
@@ -811,40 +851,12 @@ void launch_column(licom_ctx *ctx, const licom_fields *f, const licom_diag *d, i
 
 int launch_step_fused(licom_ctx *ctx, const licom_fields *f, const licom_diag *d, int flags,
                       const Scratch &s) {
-    const KGrid &g = ctx->g;
-    hipStream_t st = ctx->stream;
     if (int rc = launch_surface(ctx, f, d, s)) return rc;
     launch_column(ctx, f, d, flags, true, s);
-    {
-        Timer t(ctx, "k_march");
-        MarchArgs a{};
-        a.at = f->at;
-        a.atb = f->atb;
-        a.akt = f->akt;
-        a.uw = s.uw;
-        a.vs = s.vs;
-        a.ws = f->ws;
-        a.stf_n = s.stf_n;
-        a.err_norm2 = s.err_norm2;
-        a.swv = f->swv;
-        a.restore = f->restore;
-        a.ori = s.ori;
-        a.ax = d ? d->ax : nullptr;
-        a.ay = d ? d->ay : nullptr;
-        a.az = d ? d->az : nullptr;
-        a.dz = d ? d->dz : nullptr;
-        a.pen = d ? d->penetrate : nullptr;
-        a.flags_out = ctx->flags_out;
-        a.ntx = (g.imt - 4 + BX - 1) / BX;
-        const int nty = (g.jmt - 4 + BY - 1) / BY;
-        a.ntiles = a.ntx * nty;
-        a.tiles_per_xcd = (a.ntiles + 7) / 8;
-        const unsigned nb = 16 * a.tiles_per_xcd;
-        switch (ctx->kp.adv) {
-            case LICOM_ADV_CENTERED: k_march<LICOM_ADV_CENTERED><<<nb, NT, 0, st>>>(g, ctx->kp, a); break;
-            case LICOM_ADV_FLUX: k_march<LICOM_ADV_FLUX><<<nb, NT, 0, st>>>(g, ctx->kp, a); break;
-            default: k_march<LICOM_ADV_TSPAS><<<nb, NT, 0, st>>>(g, ctx->kp, a); break;
-        }
+    switch (ctx->kp.adv) {
+        case LICOM_ADV_CENTERED: launch_update<LICOM_ADV_CENTERED>(ctx, f, d, s); break;
+        case LICOM_ADV_FLUX: launch_update<LICOM_ADV_FLUX>(ctx, f, d, s); break;
+        default: launch_update<LICOM_ADV_TSPAS>(ctx, f, d, s); break;
     }
     launch_column(ctx, f, d, flags, false, s);
     if (flags & LICOM_STEP_SIDE_EFFECTS) launch_side(ctx, f);

@@ -67,7 +67,7 @@ struct licom_ctx {
     // licomqice [jmt][imt] (device) written by steps with LICOM_STEP_ICESNOW
     double *qice = nullptr;
     // tspas limiter flags [2][km][jmt][imt] (device, 1 byte) written by the
-    // fused FP64 and mixed k-marches when set (licom_tracer_set_flag_output)
+    // FP64 update and the mixed k-march when set (licom_tracer_set_flag_output)
     uint8_t *flags_out = nullptr;
     licom::KGrid g{};
     licom::KPar kp{};
@@ -107,7 +107,7 @@ int launch_icesnow(licom_ctx *ctx, double *at, double *qice, int reset);
 // shared pieces of tracer_kernels.hip used by both paths
 int launch_surface(licom_ctx *ctx, const licom_fields *f, const licom_diag *d, const Scratch &s);
 int launch_halo(licom_ctx *ctx, const licom_fields *f, int flags);
-// tracer_fused.hip: prelude / k-march / column solve (production path)
+// tracer_fused.hip: prelude / flags / update / column solve (production path)
 // s: the step's scratch (the context's, or the no-allocation entry point's)
 int launch_step_fused(licom_ctx *ctx, const licom_fields *f, const licom_diag *d, int flags,
                       const Scratch &s);

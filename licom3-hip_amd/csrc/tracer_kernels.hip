@@ -150,7 +150,8 @@ __device__ __forceinline__ void predictor_terms(const KGrid &g, double dts, cons
     const double Wk = W[c], Wb = k < g.km - 1 ? W[c + sk] : 0.0;
     dev::pterms(T[c], T[c + 1], T[c - 1], T[c + sj], T[c - sj], Tu, Td, U[c + 1], U[c], V[c],
                 V[c - sj], Wk, Wb, g.tarea_r[q], g.htw[q + 1] * g.hun[q + 1], g.htw[q] * g.hun[q],
-                g.hts[q] * g.hue[q], g.hts[q - sj] * g.hue[q - sj], k, g.km, g.odzp, g.odzt, dts, t);
+                g.hts[q] * g.hue[q], g.hts[q - sj] * g.hue[q - sj], k, g.km, g.odzp[k],
+                g.odzt[k], k < g.km - 1 ? g.odzt[k + 1] : 0.0, dts, t);
 }
 
 // Value entering the 7-point bounds: at on ocean cells, the sentinel on land
@@ -270,7 +271,7 @@ __global__ void k_correct(KGrid g, KPar p, const double *__restrict__ at,
             const double Wb = k < km - 1 ? ws[c + n2] : 0.0;
             const dev::CFAdv r = dev::adv_cf(p.adv, Tc, T[c + 1], T[c - 1], T[c + sj], T[c - sj], Tu, Td,
                                              uw[c + 1], uw[c], vs[c], vs[c - sj], ws[c], Wb,
-                                             g.tarea_r[q], k, km, odzp);
+                                             g.tarea_r[q], k, km, odzp[k]);
             if (p.adv == LICOM_ADV_CENTERED) {
                 const double nss = (double)p.nss;
                 if (ax) ax[n * n3 + c] = ax[n * n3 + c] + r.hx / nss;

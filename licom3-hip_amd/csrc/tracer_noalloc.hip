@@ -6,7 +6,8 @@
 // The array (kNoallocBytes) holds the scratch of grids up to
 // 32 * imt*jmt*km + 44 * imt*jmt bytes (about 4.7 M cells at km = 55, e.g.
 // 360 x 218 x 55): the face velocities u_wface/v_sface, the explicit update
-// of both tracers, the surface and SSSNORM fields and the mixing counter.
+// of both tracers, the surface and SSSNORM fields and the mixing counter,
+// followed by the limiter flags (kFlagBytes more, 2 bytes a cell).
 // Each device the library runs on holds one copy until the process ends.
 // Every call on a device shares that device's copy: calls that overlap on
 // one device (several streams or threads) race.  Each call clears the part
@@ -25,7 +26,10 @@ namespace {
 constexpr size_t kNoallocBytes = size_t(160) << 20;
 constexpr int kMaxDevices = 64;
 
-__device__ __align__(256) unsigned char scratch[kNoallocBytes];
+// 2 of every 32 bytes, rounded up
+constexpr size_t kFlagBytes = kNoallocBytes / 16 + 256;
+
+__device__ __align__(256) unsigned char scratch[kNoallocBytes + kFlagBytes];
 
 std::mutex g_mu;
 void *g_ptr[kMaxDevices] = {};       // device address of `scratch`, per device
@@ -39,7 +43,8 @@ __global__ __launch_bounds__(256) void k_zero16(uint4 *p, size_t n) {
 size_t al256(size_t b) { return (b + 255) & ~size_t(255); }
 
 // Carves the scratch of one step out of base (NULL: sizes only); returns
-// the bytes used.
+// the bytes used in front of the flags, which every step writes before it
+// reads them.
 size_t carve(const licom_ctx *c, unsigned char *base, Scratch &s) {
     const size_t n2 = c->n2, n3 = c->n3;
     size_t off = 0;
@@ -57,10 +62,11 @@ size_t carve(const licom_ctx *c, unsigned char *base, Scratch &s) {
     take(&s.vs, n3 * 8);
     take(&s.ori, 2 * n3 * 8);
     take(&s.mix_count, 8);
-    s.flags = nullptr;
+    const size_t need = off;
+    take(&s.flags, 2 * n3);
     s.d2tk = nullptr;
     s.nblk = c->s.nblk;
-    return off;
+    return need;
 }
 
 }  // namespace
@@ -89,7 +95,9 @@ extern "C" int licom_tracer_step_noalloc(licom_ctx *c, const licom_fields *f, co
                                          int flags) {
     bool split = false;
     if (int rc = plan_step(c, f, flags, split, "licom_tracer_step_noalloc")) return rc;
-    if (flags & LICOM_STEP_STAGED) {
+    const uintptr_t al = reinterpret_cast<uintptr_t>(f->at) | reinterpret_cast<uintptr_t>(f->atb) |
+                         reinterpret_cast<uintptr_t>(f->ws) | reinterpret_cast<uintptr_t>(f->akt);
+    if ((flags & LICOM_STEP_STAGED) || c->imt % 2 != 0 || (al & 15) != 0) {
         set_error("licom_tracer_step_noalloc runs the fused kernels only: it needs an even imt, "
                   "16-byte aligned at/atb/ws/akt, no LICOM_STEP_STAGED and not ICESNOW with "
                   "VTL_SCRATCH");
