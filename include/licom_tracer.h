@@ -217,8 +217,7 @@ int licom_tracer_step_mixed(licom_ctx *ctx, const licom_fields_mixed *f,
 /* ---- Batched ensemble engine (mixed-precision form) --------------------
  * Advances many members, each a context of its own grid (any size), in one
  * launch per stage and step: every stage kernel walks a work list of
- * (member, block) items; the k-march runs persistent workgroups over
- * (member, tile, tracer) items.  A member's results are bit-identical
+ * (member, block) items.  A member's results are bit-identical
  * whether it runs alone (licom_tracer_step_mixed), in any batch, or under
  * any launch-shape choice.  No reference counterpart (the reference runs one
  * domain per rank). */
@@ -241,13 +240,14 @@ int licom_batch_create(licom_ctx *const *members, const licom_fields_mixed *fiel
                        const licom_diag_mixed *diags, const licom_member_tuning *tuning,
                        int n, licom_batch **out);
 int licom_batch_set_stream(licom_batch *b, void *hip_stream);
-/* Workgroups of the persistent k-march; 0 = one workgroup per item. */
+/* Workgroups of the update, which stride through its items; 0 = one
+ * workgroup per item. */
 int licom_batch_set_march_grid(licom_batch *b, int workgroups);
 /* on != 0: each step is ONE launch (steps and captured graphs alike): a
  * grid of co-resident workgroups (occupancy x CUs) walks every stage's work
  * list, with a grid-wide barrier between dependent phases (surface |
- * SSSNORM partials | SSSNORM total + prelude | k-march | solve | side effects
- * + halo).  Same results bit for bit as the default of one launch per stage.
+ * SSSNORM partials | SSSNORM total + prelude | limiter flags | update |
+ * solve | side effects + halo).  Same results bit for bit as the default of one launch per stage.
  * The barrier waits are bounded: if the workgroups cannot all be resident
  * (other work sharing the device) a wait times out after about a second and
  * licom_batch_sync returns LICOM_EHIP (the members' state is then

@@ -2,7 +2,7 @@
 //
 // The tracer state (at, atb), the surface fields, the implicit vertical solve,
 // convadj and the SSSNORM sum stay FP64; velocities, ws, akt, the face
-// velocities, the divergence and the 3-D diagnostics are FP32.  The k-march
+// velocities, the divergence and the 3-D diagnostics are FP32.  The update
 // forms every difference of the tracer (neighbour minus the cell's own value)
 // in FP64 and runs the tspas fluxes, the limiter test, the del4/del2 stencils
 // and the explicit vertical diffusion in FP32 on those anomalies; its FP32
@@ -13,7 +13,8 @@
 // increments.
 //
 //   k_prelude_mx<KM>              face velocities, divergence, continuity w
-//   k_march_mx                    four-wave k-march (as the FP64 k_march)
+//   k_flags_mx / k_update_mx      limiter flags and explicit update (as the FP64
+//                                 k_flags / k_update)
 //   k_solve<KM, float, float>     FP64 invtrit + convadj (tracer_solve.h)
 //   k_side3<float4> / k_side2_mx  in-place side effects
 #include <hip/hip_runtime.h>
@@ -21,6 +22,7 @@
 #include <algorithm>
 #include <vector>
 
+#include "tracer_cells.h"
 #include "tracer_device.h"
 #include "tracer_internal.h"
 #include "tracer_solve.h"
@@ -182,82 +184,42 @@ __global__ __launch_bounds__(256) void k_prelude_mx(KGrid g, float oncc, const f
     prelude_col_mx_body<KM>(g, oncc, utf, utl, vtf, vtl, work_u, stf_pre, ws, uw, vs, bx, by, shape);
 }
 
-// --------------------------------------------------------------- march
-// A 32x6 tile: each of the three tile waves owns two whole 32-cell rows, so
-// that the level's FP32 stores leave in 128-byte row pieces (the march is
-// bound by its scattered stores, and the 64-byte pieces of a 16-wide tile
-// cost a third more time). Wave 3 is the ring/staging wave: its lane l
-// takes ring cell l (the north and south rows) and, for l < 12, ring cell
-// 64 + l (the west and east columns). Workgroups of four waves: with five
-// or six, residency fell to under two workgroups per CU.
-constexpr int BX = 32, BY = 6;
-constexpr int PX = BX + 2, PY = BY + 2;
-constexpr int RX = BX + 4, RY = BY + 4;
-constexpr int NOWN = BX * BY, NRING = 2 * (BX + BY), NT = NOWN + 64;
-static_assert(NOWN == 192 && 2 * BX == 64 && NRING > 64 && NRING <= 128,
-              "three tile waves; one ring wave with a second ring cell on its first lanes");
-constexpr int NP = PX * PY, NR = RX * RY;
-constexpr int NCH = NR / 2, NCI = (NCH + 63) / 64;   // 16-byte chunks of an FP64 window
-constexpr int NCF = (NR + 63) / 64;                  // dword loads of an FP32 window
-constexpr int NCA = NOWN / 64;                       // dword loads of the tile's akt
-constexpr int MARCH_BLOCKS = 3;                      // resident workgroups per CU (LDS)
+// --------------------------------------------------- limiter flags and update
+// As the FP64 k_flags / k_update (tracer_fused.hip): two cells a lane, DPP
+// neighbours, metrics in LDS.
 constexpr float BIG = 1.0e10f;
-// Look-ahead of the staged planes (as in the FP64 k_march): at and ws are
-// issued for level k+LA+2 at the start of P(k); faces, atb, akt for k+LA+1.
-constexpr int LA = 2;
-constexpr int NAT = LA + 3, NW = LA + 3, NUV = LA + 2, NB = LA + 2;
-constexpr int DMA_ATW = NCI + NCF;                  // at (16-byte), ws (dword)
-constexpr int DMA_UVBA = 2 * NCF + NCI + NCA;       // u, v (dword), atb (16-byte), akt (dword)
 
-struct MarchArgsMx {
+struct F2 {
+    float v[2];
+};
+typedef float licom_f2 __attribute__((ext_vector_type(2), aligned(4)));
+typedef float licom_f2a __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ F2 ld2(const float *plane, uint32_t off) {
+    const licom_f2 x = *reinterpret_cast<const licom_f2 *>(reinterpret_cast<const char *>(plane) + off);
+    return F2{{x.x, x.y}};
+}
+__device__ __forceinline__ void st2(float *plane, uint32_t off, const float (&x)[2], bool a0, bool a1) {
+    char *p = reinterpret_cast<char *>(plane) + off;
+    if (a0 && a1) {
+        *reinterpret_cast<licom_f2 *>(p) = licom_f2{x[0], x[1]};
+    } else if (a0 || a1) {
+        *reinterpret_cast<float *>(p + (a0 ? 0 : 4)) = a0 ? x[0] : x[1];
+    }
+}
+template <int CTRL>
+__device__ __forceinline__ float dppf(float x) {
+    return __builtin_bit_cast(float, dpp<CTRL>(__builtin_bit_cast(int, x)));
+}
+__device__ __forceinline__ F2 west(const F2 &x) { return F2{{dppf<kFromPrev>(x.v[1]), x.v[0]}}; }
+__device__ __forceinline__ F2 east(const F2 &x) { return F2{{x.v[1], dppf<kFromNext>(x.v[0])}}; }
+
+struct CellsMx {
     const double *at, *atb, *stf_n, *err_norm2, *swv, *restore;
     const float *akt, *uw, *vs, *ws;
     double *ori;
     float *ax, *ay, *az, *dz, *pen;
-    uint8_t *flags_out = nullptr;   // the limiter flag of every physical cell, or NULL
-    int ntx, ntiles, tiles_per_xcd;
-};
-
-// Ring cell r (0..NRING-1) -> P-plane coordinates (pi, pj): north row, south
-// row, west column, east column, corners excluded.
-__device__ __forceinline__ int2 ring_cell(int r) {
-    const bool ns = r < 2 * BX;
-    const int rr = ns ? r : r - 2 * BX;
-    const int pi = ns ? 1 + (rr % BX) : (rr < BY ? 0 : PX - 1);
-    const int pj = ns ? (rr < BX ? 0 : PY - 1) : 1 + (rr % BY);
-    return make_int2(pi, pj);
-}
-
-// FP32 metrics of a cell: tarea_r, the LW coefficients 2 dts tarea_r / D
-// (D = htw*hun at i+1, i; hts*hue at j, j-1) and the del2 stencil.
-struct MetricsF {
-    float tr, cx1, cx2, cx3, cx4, dtn, dts, dte, dtw, ahf;
-};
-
-__device__ __forceinline__ MetricsF load_metrics_f(const KGrid &g, int gj, int gi, double dts) {
-    const size_t q = (size_t)gj * g.imt + gi, sj = g.imt;
-    const double tr = g.tarea_r[q];
-    MetricsF m;
-    m.tr = (float)tr;
-    m.cx1 = (float)(2.0 * dts * tr / (g.htw[q + 1] * g.hun[q + 1]));
-    m.cx2 = (float)(2.0 * dts * tr / (g.htw[q] * g.hun[q]));
-    m.cx3 = (float)(2.0 * dts * tr / (g.hts[q] * g.hue[q]));
-    m.cx4 = (float)(2.0 * dts * tr / (g.hts[q - sj] * g.hue[q - sj]));
-    m.dtn = (float)g.dtn[q];
-    m.dts = (float)g.dts[q];
-    m.dte = (float)g.dte[q];
-    m.dtw = (float)g.dtw[q];
-    m.ahf = (float)g.ahf[q];
-    return m;
-}
-
-struct LWf {
-    float xy1, xy2, xy3, xy4, zb1, zb2;
-};
-
-struct LvM {
-    const double *Pk, *Pu, *Pd;
-    const float *U, *V, *Wk, *Wb;
+    uint8_t *flags;
+    uint8_t *flags_out;   // the limiter flag of every physical cell, or NULL
 };
 
 // Anomalies of the six neighbours about the cell value (FP64 differences).
@@ -275,435 +237,408 @@ __device__ __forceinline__ void cheap_mx(const Anom &a, float Ue, float Uw, floa
     zc = 0.5f * odzpk * (Wk * a.u - Wb * a.d);
 }
 
-// Predictor and limiter flag of level K at R-plane index r (mixed form).
-__device__ __forceinline__ bool pred_flag_mx(const KGrid &g, int r, const LvM &L, const int *sK,
-                                             int K, const float *odzp, const float *odzt, float dts,
-                                             const MetricsF &M, LWf &lw) {
-    const int km = g.km;
-    const double Tc = L.Pk[r];
+struct LWf {
+    float xy1, xy2, xy3, xy4, zb1, zb2;
+};
+// The Lax-Wendroff terms; cx: 2 dts tarea_r / D (D = htw*hun at i+1, i;
+// hts*hue at j, j-1).
+__device__ __forceinline__ LWf lw_mx(const Anom &a, float Ue, float Uw, float Vs, float Vn, float Wk, float Wb,
+                                     float oz, float ot, float ot1, float dts, float cx1, float cx2, float cx3,
+                                     float cx4, bool top, bool bot) {
+    LWf l;
+    l.xy1 = -(a.e * Ue * Ue) * cx1;
+    l.xy2 = -(a.w * Uw * Uw) * cx2;
+    l.xy3 = -(a.s * Vs * Vs) * cx3;
+    l.xy4 = -(a.n * Vn * Vn) * cx4;
+    l.zb1 = top ? 0.0f : -0.5f * oz * Wk * Wk * ot * a.u * dts;
+    l.zb2 = bot ? 0.0f : -0.5f * oz * Wb * Wb * ot1 * a.d * dts;
+    return l;
+}
+
+// tarea_r and the Lax-Wendroff coefficients of a lane's two cells.
+struct FacesF {
+    F2 tr, cx1, cx2, cx3, cx4;
+};
+__device__ __forceinline__ FacesF load_faces_f(const KGrid &g, int pc, int pn, double dts) {
+    const Faces f = load_faces(g, pc, pn);
+    FacesF r;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        const double c = 2.0 * dts * f.tr[e];
+        r.tr.v[e] = (float)f.tr[e];
+        r.cx1.v[e] = (float)(c / f.dx[e + 1]);
+        r.cx2.v[e] = (float)(c / f.dx[e]);
+        r.cx3.v[e] = (float)(c / f.ds[e]);
+        r.cx4.v[e] = (float)(c / f.dn[e]);
+    }
+    return r;
+}
+
+// Anomalies of cell e of a lane.
+__device__ __forceinline__ Anom anom(int e, const D2 &Tc, const D2 &Te, const D2 &Tw, const D2 &Ts, const D2 &Tn,
+                                     const D2 &Tu, const D2 &Td, bool top, bool bot) {
+    const double tc = Tc.v[e];
     Anom a;
-    a.e = (float)(L.Pk[r + 1] - Tc);
-    a.w = (float)(L.Pk[r - 1] - Tc);
-    a.s = (float)(L.Pk[r + RX] - Tc);
-    a.n = (float)(L.Pk[r - RX] - Tc);
-    a.u = K > 0 ? (float)(L.Pu[r] - Tc) : 0.0f;
-    a.d = K < km - 1 ? (float)(L.Pd[r] - Tc) : 0.0f;
-    const float Ue = L.U[r + 1], Uw = L.U[r], Vs = L.V[r], Vn = L.V[r - RX];
-    const float Wk = K > 0 ? L.Wk[r] : 0.0f, Wb = K < km - 1 ? L.Wb[r] : 0.0f;
-    const float odzpk = odzp[K];
-    float xc, yc, zc;
-    cheap_mx(a, Ue, Uw, Vs, Vn, Wk, Wb, M.tr, odzpk, xc, yc, zc);
-    lw.xy1 = -(a.e * Ue * Ue) * M.cx1;
-    lw.xy2 = -(a.w * Uw * Uw) * M.cx2;
-    lw.xy3 = -(a.s * Vs * Vs) * M.cx3;
-    lw.xy4 = -(a.n * Vn * Vn) * M.cx4;
-    lw.zb1 = K > 0 ? -0.5f * odzpk * Wk * Wk * odzt[K] * a.u * dts : 0.0f;
-    lw.zb2 = K < km - 1 ? -0.5f * odzpk * Wb * Wb * odzt[K + 1] * a.d * dts : 0.0f;
-    const float xx = -(xc + lw.xy1 + lw.xy2);
-    const float yy = -(yc + lw.xy3 + lw.xy4);
-    const float zz = -(lw.zb1 + lw.zb2 + zc);
-    const float d00 = (xx + yy + zz) * dts;
-    // 7-point bounds about the cell value, land at -+1e10 (tracer.cpp:416-545)
-    float mx = sK[r] > K ? 0.0f : -BIG, mn = sK[r] > K ? 0.0f : BIG;
-    const int nb[4] = {r - RX, r + RX, r - 1, r + 1};
-    const float tv[4] = {a.n, a.s, a.w, a.e};
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-        const bool wet = sK[nb[m]] > K;
-        mx = fmaxf(mx, wet ? tv[m] : -BIG);
-        mn = fminf(mn, wet ? tv[m] : BIG);
-    }
-    if (K > 0) {
-        const bool wet = sK[r] > K - 1;
-        mx = fmaxf(mx, wet ? a.u : -BIG);
-        mn = fminf(mn, wet ? a.u : BIG);
-    }
-    if (K < km - 1) {
-        const bool wet = sK[r] > K + 1;
-        mx = fmaxf(mx, wet ? a.d : -BIG);
-        mn = fminf(mn, wet ? a.d : BIG);
-    }
-    return d00 > mx || d00 < mn;
+    a.e = (float)(Te.v[e] - tc);
+    a.w = (float)(Tw.v[e] - tc);
+    a.s = (float)(Ts.v[e] - tc);
+    a.n = (float)(Tn.v[e] - tc);
+    a.u = top ? 0.0f : (float)(Tu.v[e] - tc);
+    a.d = bot ? 0.0f : (float)(Td.v[e] - tc);
+    return a;
 }
 
-// del4 first pass, anomaly form: AHF * sum over wet neighbours of DT*(B_nbr - B).
-__device__ __forceinline__ float d2tk_mx(int r, const double *B, const int *sK, int k,
-                                         const MetricsF &M) {
+// tspas predictor and limiter flag (mixed form), one byte per cell; item: see
+// flat_item.
+__device__ __forceinline__ void flags_mx_body(const KGrid &g, double dts, const CellsMx &a, const FlatGrid &fg,
+                                              int item) {
+    int n, blk, k0;
+    flat_item(fg, item, n, blk, k0);
+    const int imt = g.imt, km = g.km, n2 = imt * g.jmt, lane = (int)threadIdx.x & 63;
+    const int p = lane_cell(fg, blk);
+    const int pc = clamp_cell(p, n2), pn = clamp_cell(p - imt, n2), ps = clamp_cell(p + imt, n2);
+    uint32_t bc = 8u * (uint32_t)pc, bn = 8u * (uint32_t)pn, bs = 8u * (uint32_t)ps;
+    const bool own = lane >= 1 && lane <= 62;
+    const bool own0 = own && p < fg.last, own1 = own && p + 1 < fg.last;
+    const double *T = a.at + (size_t)n * n2 * km;
+    uint8_t *F = a.flags + (size_t)n * n2 * km;
+    const float dtsf = (float)dts;
+    const FacesF M = load_faces_f(g, pc, pn, dts);
+    int kc[4], kn[2], ks[2];     // wet levels: cells -1..2, and the rows beside
+    kc[1] = g.kmt[pc];
+    kc[2] = g.kmt[pc + 1];
+    kc[0] = dpp<kFromPrev>(kc[2]);
+    kc[3] = dpp<kFromNext>(kc[1]);
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        kn[e] = g.kmt[pn + e];
+        ks[e] = g.kmt[ps + e];
+    }
+    const int k1 = min(k0 + fg.kc, km);
+    const size_t o0 = (size_t)k0 * n2;
+    D2 Tu{}, Tc = ld2(T + o0, bc);
+    F2 Wk = ld2(a.ws + o0, bc >> 1);
+    if (k0 > 0) Tu = ld2(T + o0 - n2, bc);
+    march_levels(k0, k1, km, [&](auto pos, int K) {
+        constexpr bool top = pos == 0, bot = pos == 2;
+        const float oz = (float)g.odzp[K], ot = (float)g.odzt[K], ot1 = bot ? 0.0f : (float)g.odzt[K + 1];
+        const size_t o = (size_t)K * n2;
+        fresh(bc);
+        fresh(bn);
+        fresh(bs);
+        const D2 Tn = ld2(T + o, bn), Ts = ld2(T + o, bs);
+        const F2 U = ld2(a.uw + o, bc >> 1), Vs = ld2(a.vs + o, bc >> 1), Vn = ld2(a.vs + o, bn >> 1);
+        D2 Td{};
+        F2 Wb{};
+        if constexpr (!bot) {
+            Td = ld2(T + o + n2, bc);
+            Wb = ld2(a.ws + o + n2, bc >> 1);
+        }
+        const D2 Tw = west(Tc), Te = east(Tc);
+        const F2 Ue = east(U);
+        uint32_t fl = 0;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const Anom an = anom(e, Tc, Te, Tw, Ts, Tn, Tu, Td, top, bot);
+            const float wk = top ? 0.0f : Wk.v[e], wb = Wb.v[e];
+            float xc, yc, zc;
+            cheap_mx(an, Ue.v[e], U.v[e], Vs.v[e], Vn.v[e], wk, wb, M.tr.v[e], oz, xc, yc, zc);
+            const LWf l = lw_mx(an, Ue.v[e], U.v[e], Vs.v[e], Vn.v[e], wk, wb, oz, ot, ot1, dtsf, M.cx1.v[e],
+                                M.cx2.v[e], M.cx3.v[e], M.cx4.v[e], top, bot);
+            const float xx = -(xc + l.xy1 + l.xy2);
+            const float yy = -(yc + l.xy3 + l.xy4);
+            const float zz = -(l.zb1 + l.zb2 + zc);
+            const float d00 = (xx + yy + zz) * dtsf;
+            // 7-point bounds about the cell value, land at -+1e10 (tracer.cpp:416-545)
+            const int kz = kc[e + 1];
+            float mx = kz > K ? 0.0f : -BIG, mn = kz > K ? 0.0f : BIG;
+            auto bound = [&](bool wet, float v) {
+                mx = fmaxf(mx, wet ? v : -BIG);
+                mn = fminf(mn, wet ? v : BIG);
+            };
+            bound(kn[e] > K, an.n);
+            bound(ks[e] > K, an.s);
+            bound(kc[e] > K, an.w);
+            bound(kc[e + 2] > K, an.e);
+            if constexpr (!top) bound(kz > K - 1, an.u);
+            if constexpr (!bot) bound(kz > K + 1, an.d);
+            fl |= (uint32_t)(d00 > mx || d00 < mn) << (8 * e);
+        }
+        const uint32_t fc8 = bc >> 3;
+        if (own1) *reinterpret_cast<licom_u16 *>(F + o + fc8) = (uint16_t)fl;
+        else if (own0) F[o + fc8] = (uint8_t)fl;
+        Tu = Tc;
+        Tc = Td;
+        Wk = Wb;
+    });
+}
+
+// del2 stencil of a lane's two cells in one row, FP32 (DTN..DTW, AHF).
+struct Del2F {
+    F2 dn, ds, de, dw;
+};
+// sum over wet neighbours of DT*(B_nbr - B), the differences in FP64
+__device__ __forceinline__ float del2_mx(const Del2F &m, uint32_t wet, int e, uint32_t k, double Bc, double Bn,
+                                         double Bs, double Be, double Bw) {
     float h = 0.0f;
-    if (k <= sK[r] - 1) {
-        const double Bc = B[r];
-        if (k <= sK[r - RX] - 1) h += M.dtn * (float)(B[r - RX] - Bc);
-        if (k <= sK[r + RX] - 1) h += M.dts * (float)(B[r + RX] - Bc);
-        if (k <= sK[r + 1] - 1) h += M.dte * (float)(B[r + 1] - Bc);
-        if (k <= sK[r - 1] - 1) h += M.dtw * (float)(B[r - 1] - Bc);
+    if (k < (wet & 255u)) h += m.dn.v[e] * (float)(Bn - Bc);
+    if (k < (wet >> 8 & 255u)) h += m.ds.v[e] * (float)(Bs - Bc);
+    if (k < (wet >> 16 & 255u)) h += m.de.v[e] * (float)(Be - Bc);
+    if (k < (wet >> 24)) h += m.dw.v[e] * (float)(Bw - Bc);
+    return h;
+}
+
+// Explicit update of a run of cells (mixed form); sM: the lanes' metrics,
+// kept here between levels.
+constexpr int kSlotsMx = 20;
+template <bool DEL4>
+__device__ __forceinline__ void update_mx_body(const KGrid &g, const KPar &p, const CellsMx &a, const FlatGrid &fg,
+                                               int item, licom_f2a (*sM)[256]) {
+    int n, blk, k0;
+    flat_item(fg, item, n, blk, k0);
+    const int imt = g.imt, km = g.km, n2 = imt * g.jmt, lane = (int)threadIdx.x & 63;
+    const size_t n3 = (size_t)n2 * km;
+    const int pl = lane_cell(fg, blk);
+    const int pc = clamp_cell(pl, n2), pn = clamp_cell(pl - imt, n2), ps = clamp_cell(pl + imt, n2);
+    uint32_t bc = 8u * (uint32_t)pc, bn = 8u * (uint32_t)pn, bs = 8u * (uint32_t)ps;
+    bool own[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        const int c = pl + e, i = c % imt;
+        own[e] = lane >= 1 && lane <= 62 && c < fg.last && i >= 2 && i < imt - 2;
     }
-    return M.ahf * h;
-}
-
-#define LDS_PTR(p) ((__attribute__((address_space(3))) void *)(p))
-
-// Direct global->LDS loads issued through inline assembly: the compiler
-// then neither reorders them nor inserts vector-memory waits before this
-// wave's later LDS reads (which touch other slots); the staging wave waits
-// for them itself (wait_vmem) before the barrier that publishes the planes.
-// M0 holds the wave's LDS destination; nothing else in these kernels uses M0.
-__device__ __forceinline__ uint32_t lds_addr(const void *p) {
-    return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)LDS_PTR(p));
-}
-__device__ __forceinline__ void dma16(const void *g, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(g)
-                 : "memory");
-}
-__device__ __forceinline__ void dma4(const void *g, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(g)
-                 : "memory");
-}
-
-__device__ __forceinline__ void stage_d(const double *src, double *dst, const int (&off)[NCI],
-                                        int lane) {
-#pragma unroll
-    for (int u = 0; u < NCI; ++u)
-        if (u * 64 + lane < NCH)
-            dma16(src + off[u], lds_addr(dst + 128 * u));
-}
-
-__device__ __forceinline__ void stage_f(const float *src, float *dst, const int (&off)[NCF],
-                                        int lane) {
-#pragma unroll
-    for (int u = 0; u < NCF; ++u)
-        if (u * 64 + lane < NR)
-            dma4(src + off[u], lds_addr(dst + 64 * u));
-}
-
-// akt of the tile (read only at the tile's own cells): NOWN floats in NCA
-// dword instructions; element c of the slot is tile lane c.
-__device__ __forceinline__ void stage_tile_f(const float *src, float *dst, const int (&off)[NCA],
-                                             int lane) {
-#pragma unroll
-    for (int u = 0; u < NCA; ++u) dma4(src + off[u], lds_addr(dst + 64 * u));
-}
-
-__device__ __forceinline__ void wait_vmem() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-template <int N>
-__device__ __forceinline__ void wait_vmem_n() {
-    static_assert(N >= 0 && N <= 63, "vmcnt range");
-    asm volatile("s_waitcnt vmcnt(%0)" ::"I"(N) : "memory");
-}
-// Waits for every staged load except the `issued` issued at the start of
-// the current level (direct-to-LDS loads complete in order): DMA_ATW +
-// DMA_UVBA, DMA_UVBA or none.
-__device__ __forceinline__ void wait_vmem_keep(int issued) {
-    if (issued == DMA_ATW + DMA_UVBA) wait_vmem_n<DMA_ATW + DMA_UVBA>();
-    else if (issued == DMA_UVBA) wait_vmem_n<DMA_UVBA>();
-    else wait_vmem_n<0>();
-}
-__device__ __forceinline__ void bar_lds() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-__device__ __forceinline__ void march_body(const KGrid &g, const KPar &p, const MarchArgsMx &a, int tile,
-                                           int n) {
-    __shared__ __align__(16) double sAT[NAT][NR];
-    __shared__ __align__(16) double sB[NB][NR];
-    __shared__ __align__(16) float sU[NUV][NR];
-    __shared__ __align__(16) float sV[NUV][NR];
-    __shared__ __align__(16) float sW[NW][NR];
-    __shared__ float sD2[NP];
-    __shared__ unsigned char sFL[2][NP];
-    __shared__ int sK[NR];
-    // per-level constants and the tile's akt come from LDS, so that no
-    // vector-memory load in the level loop carries a vmcnt wait (on gfx9
-    // vmcnt also covers the staged planes and the level's stores)
-    __shared__ float sZP[KMAXM], sZT[KMAXM], sPN[KMAXM];
-    __shared__ __align__(16) float sAK[NB][NOWN];
-
-    const int imt = g.imt, jmt = g.jmt, km = g.km;
-    const size_t n2 = (size_t)imt * jmt, n3 = n2 * km;
-    const int gi0 = 2 + (tile % a.ntx) * BX, gj0 = 2 + (tile / a.ntx) * BY;
-    const long e0 = (long)(gj0 - 2) * imt + (gi0 - 2);
-
-    const int t = threadIdx.x, lane = t & 63;
-    // wave 3 (lanes NOWN..NT-1) is the ring/staging wave; the test goes
-    // through a scalar register so that the two roles compile to two
-    // separate loops behind a uniform branch (with a per-lane test they are
-    // merged into one exec-masked loop, and the tile waves' loads and stores
-    // then carry vmcnt waits into the staging wave's code)
-    const bool ringw = __builtin_amdgcn_readfirstlane(t >> 6) == NOWN / 64;
-    const int2 rc = ring_cell(ringw ? t - NOWN : 0);   // ring cell `lane` (< 64 < NRING)
-    const int pi = ringw ? rc.x : 1 + t % BX, pj = ringw ? rc.y : 1 + t / BX;
-    const int gi = gi0 - 1 + pi, gj = gj0 - 1 + pj;
-    const int rC = (pj + 1) * RX + (pi + 1), pC = pj * PX + pi;
-    const bool cell_ok = gj >= 1 && gj < jmt - 1 && gi >= 1 && gi < imt - 1;
-    const bool act = !ringw && gi < imt - 2 && gj < jmt - 2;
-    const size_t q = cell_ok ? (size_t)gj * imt + gi : 0;
-
     const double *T = a.at + n * n3;
     const double *TB = a.atb + n * (n3 + n2) + n2;
     const float *A = a.akt + n * n3;
+    const uint8_t *F = a.flags + n * n3;
     const double dts = p.dts;
-    const float dtsf = (float)dts;
-
-    for (int r = t; r < NR; r += NT) {
-        const int rj = gj0 - 2 + r / RX, ri = gi0 - 2 + r % RX;
-        sK[r] = (rj < jmt && ri < imt) ? g.kmt[(size_t)rj * imt + ri] : 0;
-    }
-    for (int r = t; r < km; r += NT) {
-        sZP[r] = (float)g.odzp[r];
-        sZT[r] = (float)g.odzt[r];
-        sPN[r] = r < km - 1 ? (float)g.pen[r] : 0.0f;
-    }
-    MetricsF M{};
-    if (cell_ok) M = load_metrics_f(g, gj, gi, dts);
-
-    if (ringw) {
-        int offd[NCI], offf[NCF];
-#pragma unroll
-        for (int u = 0; u < NCI; ++u) {
-            const int c = min(u * 64 + lane, NCH - 1), row = c / (RX / 2), cp = c - row * (RX / 2);
-            offd[u] = (int)min(e0 + (long)row * imt + 2 * cp, (long)n2 - 2);
-        }
-#pragma unroll
-        for (int u = 0; u < NCF; ++u) {
-            const int c = min(u * 64 + lane, NR - 1), row = c / RX, col = c - row * RX;
-            offf[u] = (int)min(e0 + (long)row * imt + col, (long)n2 - 1);
-        }
-        int offa[NCA];
-#pragma unroll
-        for (int u = 0; u < NCA; ++u) {
-            const int c = u * 64 + lane, row = c / BX, col = c - row * BX;
-            offa[u] = (int)min((long)(gj0 + row) * imt + gi0 + col, (long)n2 - 1);
-        }
-        for (int l = 0; l < NAT - 1 && l < km; ++l) {
-            stage_d(T + (size_t)l * n2, sAT[l], offd, lane);
-            stage_f(a.ws + (size_t)l * n2, sW[l], offf, lane);
-        }
-        for (int l = 0; l < NUV - 1 && l < km; ++l) {
-            stage_f(a.uw + (size_t)l * n2, sU[l], offf, lane);
-            stage_f(a.vs + (size_t)l * n2, sV[l], offf, lane);
-            stage_d(TB + (size_t)l * n2, sB[l], offd, lane);
-            stage_tile_f(A + (size_t)l * n2, sAK[l], offa, lane);
-        }
-        // the second ring cell of lanes 0..NRING-65 (west and east columns)
-        const bool hasB = lane < NRING - 64;
-        const int2 rb = ring_cell(hasB ? 64 + lane : 64);
-        const int giB = gi0 - 1 + rb.x, gjB = gj0 - 1 + rb.y;
-        const int rCB = (rb.y + 1) * RX + (rb.x + 1), pCB = rb.y * PX + rb.x;
-        const bool okB = hasB && gjB >= 1 && gjB < jmt - 1 && giB >= 1 && giB < imt - 1;
-        // their metrics live in LDS: in registers they push the persistent
-        // ensemble march over its register budget
-        __shared__ MetricsF sMB[NRING - 64];
-        const MetricsF &MB = sMB[min(lane, NRING - 65)];
-        if (okB) sMB[lane] = load_metrics_f(g, gjB, giB, dts);
-        wait_vmem();
-        bar_lds();
-        {
-            LWf tmp;
-            const LvM L0{sAT[0], sAT[0], sAT[1], sU[0], sV[0], sW[0], sW[1]};
-            const bool f0 = cell_ok ? pred_flag_mx(g, rC, L0, sK, 0, sZP, sZT, dtsf, M, tmp) : false;
-            sFL[0][pC] = f0;
-            if (hasB) sFL[0][pCB] = okB ? pred_flag_mx(g, rCB, L0, sK, 0, sZP, sZT, dtsf, MB, tmp) : false;
-        }
-        bar_lds();
-        for (int k = 0; k < km; ++k) {
-            const int s0 = k % NAT, s1 = (k + 1) % NAT, s2 = (k + 2) % NAT, s3 = (k + LA + 2) % NAT;
-            const int u0 = k % NUV, u1 = (k + 1) % NUV, u2 = (k + LA + 1) % NUV;
-            int issued = 0;
-            if (k + LA + 2 < km) {
-                stage_d(T + (size_t)(k + LA + 2) * n2, sAT[s3], offd, lane);
-                stage_f(a.ws + (size_t)(k + LA + 2) * n2, sW[s3], offf, lane);
-                issued += DMA_ATW;
-            }
-            if (k + LA + 1 < km) {
-                stage_f(a.uw + (size_t)(k + LA + 1) * n2, sU[u2], offf, lane);
-                stage_f(a.vs + (size_t)(k + LA + 1) * n2, sV[u2], offf, lane);
-                stage_d(TB + (size_t)(k + LA + 1) * n2, sB[u2], offd, lane);
-                stage_tile_f(A + (size_t)(k + LA + 1) * n2, sAK[u2], offa, lane);
-                issued += DMA_UVBA;
-            }
-            const LvM L1{sAT[s1], sAT[s0], sAT[s2], sU[u1], sV[u1], sW[s1], sW[s2]};
-            if (k + 1 < km) {
-                LWf tmp;
-                sFL[(k + 1) & 1][pC] = cell_ok ? pred_flag_mx(g, rC, L1, sK, k + 1, sZP, sZT, dtsf, M, tmp) : false;
-            }
-            if (p.hmix == LICOM_HMIX_DEL4) {
-                sD2[pC] = cell_ok ? d2tk_mx(rC, sB[u0], sK, k, M) : 0.0f;
-                if (hasB) sD2[pCB] = okB ? d2tk_mx(rCB, sB[u0], sK, k, MB) : 0.0f;
-            }
-            bar_lds();
-            // C(k): the column cells' flags of level k+1, first read in
-            // C(k+1); the planes they read (at k..k+2, faces and ws of k+1)
-            // are complete and not restaged before the end of level k
-            if (k + 1 < km && hasB) {
-                LWf tmp;
-                sFL[(k + 1) & 1][pCB] = okB ? pred_flag_mx(g, rCB, L1, sK, k + 1, sZP, sZT, dtsf, MB, tmp) : false;
-            }
-            wait_vmem_keep(issued);
-            bar_lds();
-        }
-        return;
-    }
-
-    const double sw = (n == 0 && act && a.swv) ? a.swv[q] : 0.0;
-    const int kmt_own = act ? g.kmt[q] : 0;
-    const double stf_n = act ? a.stf_n[n * n2 + q] : 0.0;
-    const double enorm = (n == 1 && p.sssnorm && act) ? a.err_norm2[0] : 0.0;
-    const bool rest = p.boundary_restore == 1 && a.restore != nullptr;
-    const double odzp0 = g.odzp[0];
-    // the per-cell loads above complete here, before the level loop, so
-    // that no wait for them (which would also wait for the level's stores)
-    // stays inside it
-    __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
-    bar_lds();
-    LWf lc{}, ln{};
+    const float dtsf = (float)dts, ah = (float)p.ah;
+    auto keep = [&](int slot, const F2 &x) { sM[slot][threadIdx.x] = licom_f2a{x.v[0], x.v[1]}; };
+    auto get = [&](int slot) {
+        const licom_f2a x = sM[slot][threadIdx.x];
+        return F2{{x.x, x.y}};
+    };
     {
-        const LvM L0{sAT[0], sAT[0], sAT[1], sU[0], sV[0], sW[0], sW[1]};
-        sFL[0][pC] = cell_ok ? pred_flag_mx(g, rC, L0, sK, 0, sZP, sZT, dtsf, M, lc) : false;
+        const FacesF M = load_faces_f(g, pc, pn, dts);
+        keep(0, M.tr);
+        keep(1, M.cx1);
+        keep(2, M.cx2);
+        keep(3, M.cx3);
+        keep(4, M.cx4);
     }
-    bar_lds();
-
-    double Tprev = 0.0, Bprev = 0.0;
-    float Aprev = 0.0f;
-    bool fprev = false;
+    uint32_t wet[3][2];
+    uint32_t bN = 0, bS = 0;
+    load_wet(g, pc, pn, ps, wet[0]);
+    if constexpr (DEL4) {
+        const int pN = clamp_cell(pl - 2 * imt, n2), pS = clamp_cell(pl + 2 * imt, n2);
+        load_wet(g, pn, pN, pc, wet[1]);
+        load_wet(g, ps, pc, pS, wet[2]);
+        bN = 8u * (uint32_t)pN;
+        bS = 8u * (uint32_t)pS;
+    }
+    {
+        const double *co[5] = {g.dtn, g.dts, g.dte, g.dtw, g.ahf};
+#pragma unroll
+        for (int r = 0; r < (DEL4 ? 3 : 1); ++r)
+#pragma unroll
+            for (int c = 0; c < (DEL4 ? 5 : 4); ++c) {
+                const int cell = r == 0 ? pc : (r == 1 ? pn : ps);
+                keep(5 + r * 5 + c, F2{{(float)co[c][cell], (float)co[c][cell + 1]}});
+            }
+    }
+    auto stencil = [&](int r) { return Del2F{get(5 + r * 5), get(6 + r * 5), get(7 + r * 5), get(8 + r * 5)}; };
+    int kmt[2];
+    float sw[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        kmt[e] = g.kmt[pc + e];
+        sw[e] = (n == 0 && a.swv) ? (float)a.swv[pc + e] : 0.0f;
+    }
+    const bool rest = p.boundary_restore == 1 && a.restore != nullptr;
     const double lamda = 1.0 / (15.0 * 86400.0);
-    const float ah = (float)p.ah;
 
-    for (int k = 0; k < km; ++k) {
-        const int s0 = k % NAT, s1 = (k + 1) % NAT, s2 = (k + 2) % NAT;
-        const int u0 = k % NUV, u1 = (k + 1) % NUV;
-        const float Acur = act ? (float)dev::floor_akt((double)sAK[u0][t], k, n, p.hmix, p.dwndmix) : 0.0f;
-        if (k + 1 < km) {
-            const LvM L1{sAT[s1], sAT[s0], sAT[s2], sU[u1], sV[u1], sW[s1], sW[s2]};
-            sFL[(k + 1) & 1][pC] = cell_ok ? pred_flag_mx(g, rC, L1, sK, k + 1, sZP, sZT, dtsf, M, ln) : false;
-        }
-        if (p.hmix == LICOM_HMIX_DEL4) sD2[pC] = cell_ok ? d2tk_mx(rC, sB[u0], sK, k, M) : 0.0f;
-        bar_lds();
-
-        if (act) {
-            const double *Pk = sAT[s0], *Pk1 = sAT[s1];
-            const double *Bk = sB[u0], *Bk1 = sB[u1];
-            const unsigned char *F = sFL[k & 1];
-            const int r = rC, pp = pC;
-            const double Tc = Pk[r];
-            Anom an;
-            an.e = (float)(Pk[r + 1] - Tc);
-            an.w = (float)(Pk[r - 1] - Tc);
-            an.s = (float)(Pk[r + RX] - Tc);
-            an.n = (float)(Pk[r - RX] - Tc);
-            an.u = k > 0 ? (float)(Tprev - Tc) : 0.0f;
-            an.d = k + 1 < km ? (float)(Pk1[r] - Tc) : 0.0f;
-            const float *U = sU[u0], *V = sV[u0];
-            const float Ue = U[r + 1], Uw = U[r], Vs = V[r], Vn = V[r - RX];
-            const float Wk = k > 0 ? sW[s0][r] : 0.0f, Wb = (k + 1 < km) ? sW[s1][r] : 0.0f;
-            const bool fc = F[pp], fe = F[pp + 1], fw = F[pp - 1], fs = F[pp + PX], fn = F[pp - PX];
-            const bool fd = (k + 1 < km) ? sFL[(k + 1) & 1][pp] : false;
-            bool up1, up2, up3, up4;
-            if (k == 0 || k == km - 1) {
-                up1 = fc || (fe && gi <= imt - 3);
-                up2 = fc || (fw && gi >= 2);
-                up3 = fc || (fs && gj <= jmt - 3);
-                up4 = fc || (fn && gj >= 2);
-            } else {
-                up1 = (fc || fe) && gi <= imt - 3;
-                up2 = (fc || fw) && gi >= 2;
-                up3 = (fc || fs) && gj <= jmt - 3;
-                up4 = (fc || fn) && gj >= 2;
-            }
-            const float tr = M.tr;
-            const float odzpk = sZP[k];
-            float xc, yc, zc;
-            cheap_mx(an, Ue, Uw, Vs, Vn, Wk, Wb, tr, odzpk, xc, yc, zc);
-            const float xy1 = up1 ? -an.e * fabsf(Ue) * tr : lc.xy1;
-            const float xy2 = up2 ? -an.w * fabsf(Uw) * tr : lc.xy2;
-            const float xy3 = up3 ? -an.s * fabsf(Vs) * tr : lc.xy3;
-            const float xy4 = up4 ? -an.n * fabsf(Vn) * tr : lc.xy4;
-            float zb1 = 0.0f, zb2 = 0.0f;
-            if (k > 0) zb1 = (fc || fprev) ? -0.5f * fabsf(Wk) * odzpk * an.u : lc.zb1;
-            if (k + 1 < km) zb2 = (fc || fd) ? -0.5f * fabsf(Wb) * odzpk * an.d : lc.zb2;
-            const float xx = -(xc + xy1 + xy2);
-            const float yy = -(yc + xy3 + xy4);
-            const float zz = -(zc + zb1 + zb2);
-            const size_t c = (size_t)k * n2 + q;
-            if (a.ax) a.ax[n * n3 + c] = xx;
-            if (a.ay) a.ay[n * n3 + c] = yy;
-            if (a.az) a.az[n * n3 + c] = zz;
-            const float vk = k < kmt_own ? 1.0f : 0.0f;
-            float tf = (xx + yy + zz) * vk;
-            // horizontal mixing (tracer_del4_2 / tracer_4)
-            {
-                float h = 0.0f;
-                if (p.hmix == LICOM_HMIX_DEL4) {
-                    if (k <= sK[r] - 1) {
-                        float cc = 0.0f;
-                        if (k <= sK[r - RX] - 1) { h += M.dtn * sD2[pp - PX]; cc -= M.dtn; }
-                        if (k <= sK[r + RX] - 1) { h += M.dts * sD2[pp + PX]; cc -= M.dts; }
-                        if (k <= sK[r + 1] - 1) { h += M.dte * sD2[pp + 1]; cc -= M.dte; }
-                        if (k <= sK[r - 1] - 1) { h += M.dtw * sD2[pp - 1]; cc -= M.dtw; }
-                        h = cc * sD2[pp] + h;
-                    }
-                } else if (k <= sK[r] - 1) {
-                    const double Bc0 = Bk[r];
-                    if (k <= sK[r - RX] - 1) h += M.dtn * (float)(Bk[r - RX] - Bc0);
-                    if (k <= sK[r + RX] - 1) h += M.dts * (float)(Bk[r + RX] - Bc0);
-                    if (k <= sK[r + 1] - 1) h += M.dte * (float)(Bk[r + 1] - Bc0);
-                    if (k <= sK[r - 1] - 1) h += M.dtw * (float)(Bk[r - 1] - Bc0);
-                }
-                tf += ah * h;
-            }
-            // shortwave penetration (T) and explicit vertical diffusion
-            const float v1 = (k + 1 < km && k + 1 < kmt_own) ? 1.0f : 0.0f;
-            if (n == 0) {
-                float pv;
-                const float swf = (float)sw;
-                if (k == 0) {
-                    pv = -swf * sPN[0] * (1 < kmt_own ? 1.0f : 0.0f) * odzpk;
-                } else if (k == km - 1) {
-                    pv = swf * sPN[km - 2] * vk * odzpk;
-                } else {
-                    pv = (swf * sPN[k - 1] * vk - swf * sPN[k] * v1) * odzpk;
-                }
-                tf += pv;
-                if (a.pen) a.pen[c] = pv;
-            }
-            const double Bc = Bk[r];
-            float dzv;
-            if (k == 0) {
-                dzv = -odzpk * Acur * (float)(Bc - Bk1[r]) * sZT[1] * v1 * 0.5f;
-            } else if (k == km - 1) {
-                dzv = odzpk * Aprev * (float)(Bprev - Bc) * sZT[km - 1] * vk * 0.5f;
-            } else {
-                const float wt1 = Aprev * (float)(Bprev - Bc) * sZT[k] * vk;
-                const float wt2 = Acur * (float)(Bc - Bk1[r]) * sZT[k + 1] * v1;
-                dzv = odzpk * (wt1 - wt2) * 0.5f;
-            }
-            tf += dzv;
-            if (a.dz) a.dz[n * n3 + c] = dzv;
-            if (a.flags_out) a.flags_out[n * n3 + c] = fc;
-            if (k == 0 && kmt_own > 0) {
-                tf += (float)(stf_n * 0.5 * odzp0);
-                if (n == 1 && p.sssnorm) tf += (float)enorm * vk;
-            } else if (k == 0 && n == 1 && p.sssnorm) {
-                tf += (float)enorm * vk;
-            }
-            if (rest && k >= 1) {
-                const double Rk = a.restore[n * n3 + c];
-                tf += vk * (float)((Rk - Bc) * lamda);
-            }
-            a.ori[n * n3 + c] = Tc + dts * (double)tf;
-            Tprev = Tc;
-            Bprev = Bc;
-            fprev = fc;
-        }
-        Aprev = Acur;
-        lc = ln;
-        bar_lds();
+    const int k1 = min(k0 + fg.kc, km);
+    const size_t o0 = (size_t)k0 * n2;
+    auto floored = [&](const float *plane, int k) {
+        F2 x = ld2(plane, bc >> 1);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) x.v[e] = (float)dev::floor_akt((double)x.v[e], k, n, p.hmix, p.dwndmix);
+        return x;
+    };
+    D2 Tu{}, Bu{}, Tc = ld2(T + o0, bc), Bc = ld2(TB + o0, bc);
+    F2 Au{}, Wk = ld2(a.ws + o0, bc >> 1);
+    uint32_t fu = 0, f0 = ldf2(F + o0, bc >> 3);
+    if (k0 > 0) {
+        Tu = ld2(T + o0 - n2, bc);
+        Bu = ld2(TB + o0 - n2, bc);
+        Au = floored(A + o0 - n2, k0 - 1);
+        fu = ldf2(F + o0 - n2, bc >> 3);
     }
+    march_levels(k0, k1, km, [&](auto pos, int k) {
+        constexpr bool top = pos == 0, bot = pos == 2;
+        const double odzp0 = g.odzp[0];
+        const float oz = (float)g.odzp[k], ot = (float)g.odzt[k], ot1 = bot ? 0.0f : (float)g.odzt[k + 1];
+        const float pe = bot ? 0.0f : (float)g.pen[k], peu = top ? 0.0f : (float)g.pen[k - 1];
+        const size_t o = (size_t)k * n2, on = n * n3 + o;
+        fresh(bc);
+        fresh(bn);
+        fresh(bs);
+        if constexpr (DEL4) {
+            fresh(bN);
+            fresh(bS);
+        }
+        const uint32_t hc = bc >> 1;
+        const D2 Tn = ld2(T + o, bn), Ts = ld2(T + o, bs);
+        const D2 Bn = ld2(TB + o, bn), Bs = ld2(TB + o, bs);
+        const F2 U = ld2(a.uw + o, hc), Vs = ld2(a.vs + o, hc), Vn = ld2(a.vs + o, bn >> 1);
+        const F2 Ac = floored(A + o, k);
+        D2 Td{}, Bd{}, BN{}, BS{}, Rk{};
+        F2 Wb{};
+        uint32_t fd = 0;
+        const uint32_t fn = ldf2(F + o, bn >> 3), fs = ldf2(F + o, bs >> 3);
+        if constexpr (DEL4) {
+            BN = ld2(TB + o, bN);
+            BS = ld2(TB + o, bS);
+        }
+        if constexpr (!bot) {
+            Td = ld2(T + o + n2, bc);
+            Bd = ld2(TB + o + n2, bc);
+            Wb = ld2(a.ws + o + n2, hc);
+            fd = ldf2(F + o + n2, bc >> 3);
+        }
+        const bool rk = !top && rest;
+        if (rk) Rk = ld2(a.restore + on, bc);
+        const D2 Tw = west(Tc), Te = east(Tc), Bw = west(Bc), Be = east(Bc);
+        const F2 Ue = east(U);
+        // horizontal mixing (tracer_del4_2 / tracer_4)
+        asm volatile("" ::: "memory");
+        const Del2F M = stencil(0);
+        float hm[2];
+        if constexpr (DEL4) {
+            const D2 Nw = west(Bn), Ne = east(Bn), Sw = west(Bs), Se = east(Bs);
+            F2 dc, dn, ds;
+            {
+                const Del2F R = stencil(1);
+                const F2 ahf = get(14);
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+                    dn.v[e] = ahf.v[e] * del2_mx(R, wet[1][e], e, k, Bn.v[e], BN.v[e], Bc.v[e], Ne.v[e], Nw.v[e]);
+            }
+            {
+                const Del2F R = stencil(2);
+                const F2 ahf = get(19);
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+                    ds.v[e] = ahf.v[e] * del2_mx(R, wet[2][e], e, k, Bs.v[e], Bc.v[e], BS.v[e], Se.v[e], Sw.v[e]);
+            }
+            const F2 ahf = get(9);
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+                dc.v[e] = ahf.v[e] * del2_mx(M, wet[0][e], e, k, Bc.v[e], Bn.v[e], Bs.v[e], Be.v[e], Bw.v[e]);
+            const F2 dw = west(dc), de = east(dc);
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                float h = 0.0f, cc = 0.0f;
+                const uint32_t w = wet[0][e], kk = (uint32_t)k;
+                if (kk < (w & 255u)) { h += M.dn.v[e] * dn.v[e]; cc -= M.dn.v[e]; }
+                if (kk < (w >> 8 & 255u)) { h += M.ds.v[e] * ds.v[e]; cc -= M.ds.v[e]; }
+                if (kk < (w >> 16 & 255u)) { h += M.de.v[e] * de.v[e]; cc -= M.de.v[e]; }
+                if (kk < (w >> 24)) { h += M.dw.v[e] * dw.v[e]; cc -= M.dw.v[e]; }
+                hm[e] = k < kmt[e] ? cc * dc.v[e] + h : 0.0f;
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+                hm[e] = del2_mx(M, wet[0][e], e, k, Bc.v[e], Bn.v[e], Bs.v[e], Be.v[e], Bw.v[e]);
+        }
+        // limiter flags of the cells to the west and east
+        const uint32_t fw = ((uint32_t)dpp<kFromPrev>((int)f0) >> 8) | (f0 << 8);
+        const uint32_t fe = (f0 >> 8) | ((uint32_t)dpp<kFromNext>((int)f0) << 8);
+        const F2 tr = get(0), cx1 = get(1), cx2 = get(2), cx3 = get(3), cx4 = get(4);
+        float xx[2], yy[2], zz[2], dzv[2], pv[2];
+        double out[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const Anom an = anom(e, Tc, Te, Tw, Ts, Tn, Tu, Td, top, bot);
+            const float ue = Ue.v[e], uw = U.v[e], vs = Vs.v[e], vn = Vn.v[e];
+            const float wk = top ? 0.0f : Wk.v[e], wb = Wb.v[e];
+            const float vk = k < kmt[e] ? 1.0f : 0.0f, v1 = (!bot && k + 1 < kmt[e]) ? 1.0f : 0.0f;
+            const bool lim = (f0 >> (8 * e)) & 1u;
+            auto up = [&](uint32_t f) { return lim || ((f >> (8 * e)) & 1u); };
+            float xc, yc, zc;
+            cheap_mx(an, ue, uw, vs, vn, wk, wb, tr.v[e], oz, xc, yc, zc);
+            const LWf l = lw_mx(an, ue, uw, vs, vn, wk, wb, oz, ot, ot1, dtsf, cx1.v[e], cx2.v[e], cx3.v[e],
+                                cx4.v[e], top, bot);
+            const float xy1 = up(fe) ? -an.e * fabsf(ue) * tr.v[e] : l.xy1;
+            const float xy2 = up(fw) ? -an.w * fabsf(uw) * tr.v[e] : l.xy2;
+            const float xy3 = up(fs) ? -an.s * fabsf(vs) * tr.v[e] : l.xy3;
+            const float xy4 = up(fn) ? -an.n * fabsf(vn) * tr.v[e] : l.xy4;
+            float zb1 = 0.0f, zb2 = 0.0f;
+            if constexpr (!top) zb1 = up(fu) ? -0.5f * fabsf(wk) * oz * an.u : l.zb1;
+            if constexpr (!bot) zb2 = up(fd) ? -0.5f * fabsf(wb) * oz * an.d : l.zb2;
+            xx[e] = -(xc + xy1 + xy2);
+            yy[e] = -(yc + xy3 + xy4);
+            zz[e] = -(zc + zb1 + zb2);
+            float tf = (xx[e] + yy[e] + zz[e]) * vk;
+            tf += ah * hm[e];
+            // shortwave penetration (T) and explicit vertical diffusion
+            if constexpr (top) pv[e] = -sw[e] * pe * (1 < kmt[e] ? 1.0f : 0.0f) * oz;
+            else if constexpr (bot) pv[e] = sw[e] * peu * vk * oz;
+            else pv[e] = (sw[e] * peu * vk - sw[e] * pe * v1) * oz;
+            tf = n == 0 ? tf + pv[e] : tf;
+            const double b = Bc.v[e];
+            if constexpr (top) {
+                dzv[e] = -oz * Ac.v[e] * (float)(b - Bd.v[e]) * ot1 * v1 * 0.5f;
+            } else if constexpr (bot) {
+                dzv[e] = oz * Au.v[e] * (float)(Bu.v[e] - b) * ot * vk * 0.5f;
+            } else {
+                const float wt1 = Au.v[e] * (float)(Bu.v[e] - b) * ot * vk;
+                const float wt2 = Ac.v[e] * (float)(b - Bd.v[e]) * ot1 * v1;
+                dzv[e] = oz * (wt1 - wt2) * 0.5f;
+            }
+            tf += dzv[e];
+            if constexpr (top) {
+                if (kmt[e] > 0) tf += (float)(a.stf_n[(size_t)n * n2 + pc + e] * 0.5 * odzp0);
+                if (n == 1 && p.sssnorm) tf += (float)a.err_norm2[0] * vk;
+            }
+            if (rk) tf += vk * (float)((Rk.v[e] - b) * lamda);
+            out[e] = Tc.v[e] + dts * (double)tf;
+        }
+        if (a.ax) st2(a.ax + on, hc, xx, own[0], own[1]);
+        if (a.ay) st2(a.ay + on, hc, yy, own[0], own[1]);
+        if (a.az) st2(a.az + on, hc, zz, own[0], own[1]);
+        if (n == 0 && a.pen) st2(a.pen + o, hc, pv, own[0], own[1]);
+        if (a.dz) st2(a.dz + on, hc, dzv, own[0], own[1]);
+        if (a.flags_out) {
+            if (own[0]) a.flags_out[on + (bc >> 3)] = (uint8_t)(f0 & 1u);
+            if (own[1]) a.flags_out[on + (bc >> 3) + 1] = (uint8_t)(f0 >> 8);
+        }
+        st2(a.ori + on, bc, out, own[0], own[1]);
+        Tu = Tc;
+        Tc = Td;
+        Bu = Bc;
+        Bc = Bd;
+        Au = Ac;
+        Wk = Wb;
+        fu = f0;
+        f0 = fd;
+    });
 }
 
-__global__ __launch_bounds__(NT, MARCH_BLOCKS) void k_march_mx(KGrid g, KPar p, MarchArgsMx a) {
-    // XCD-aware placement: consecutive blocks of one XCD take the T and S
-    // halves of one tile, then the next tile of the same row of tiles.
-    const int Lb = blockIdx.x, xcd = Lb & 7, slot = Lb >> 3;
-    const int tile = xcd * a.tiles_per_xcd + (slot >> 1);
-    if (tile >= a.ntiles) return;
-    march_body(g, p, a, tile, slot & 1);
+// Two waves per SIMD for the update: at three, del4 spills 28 registers a lane
+// (4.43 against 3.65 ms at 1800 x 1151 x 55).  Both kernels there: 4.7 ms
+// (4.9 for the tile march they replace); 96 x 64 x 55 del2: 21 us (116);
+// 16 members of uneven sizes: 1.24 ms a step (1.42).
+__global__ __launch_bounds__(256, 4) void k_flags_mx(KGrid g, double dts, CellsMx a, FlatGrid fg) {
+    const int item = xcd_item((int)blockIdx.x, fg.per);
+    if (item < fg.total) flags_mx_body(g, dts, a, fg, item);
+}
+
+template <bool DEL4>
+__global__ __launch_bounds__(256, 2) void k_update_mx(KGrid g, KPar p, CellsMx a, FlatGrid fg) {
+    __shared__ licom_f2a sM[kSlotsMx][256];
+    const int item = xcd_item((int)blockIdx.x, fg.per);
+    if (item < fg.total) update_mx_body<DEL4>(g, p, a, fg, item, sM);
 }
 
 // --------------------------------------------------------------- side
@@ -802,7 +737,7 @@ int launch_step_mixed(licom_ctx *ctx, const licom_fields_mixed *f, const licom_d
     launch_column_mx(ctx, f, d, flags, true);
     {
         Timer t(ctx, "k_march");
-        MarchArgsMx a{};
+        CellsMx a{};
         a.at = f->at;
         a.atb = f->atb;
         a.akt = f->akt;
@@ -819,12 +754,13 @@ int launch_step_mixed(licom_ctx *ctx, const licom_fields_mixed *f, const licom_d
         a.az = d ? d->az : nullptr;
         a.dz = d ? d->dz : nullptr;
         a.pen = d ? d->penetrate : nullptr;
+        a.flags = s.flags;
         a.flags_out = ctx->flags_out;
-        a.ntx = (g.imt - 4 + BX - 1) / BX;
-        const int nty = (g.jmt - 4 + BY - 1) / BY;
-        a.ntiles = a.ntx * nty;
-        a.tiles_per_xcd = (a.ntiles + 7) / 8;
-        k_march_mx<<<16 * a.tiles_per_xcd, NT, 0, st>>>(g, ctx->kp, a);
+        const FlatGrid ff = flat_grid(g.imt, (g.jmt - 1) * g.imt, g.km);
+        k_flags_mx<<<8 * ff.per, 256, 0, st>>>(g, ctx->kp.dts, a, ff);
+        const FlatGrid fu = flat_grid(2 * g.imt, (g.jmt - 2) * g.imt, g.km);
+        if (ctx->kp.hmix == LICOM_HMIX_DEL4) k_update_mx<true><<<8 * fu.per, 256, 0, st>>>(g, ctx->kp, a, fu);
+        else k_update_mx<false><<<8 * fu.per, 256, 0, st>>>(g, ctx->kp, a, fu);
     }
     launch_column_mx(ctx, f, d, flags, false);
     if (flags & LICOM_STEP_SIDE_EFFECTS) {
@@ -862,6 +798,7 @@ struct MemberDev {
     double *net, *fw_norm2;
     double *stf_pre, *work_u, *stf_n, *temp11, *partials, *err_norm2, *ori;
     float *uw, *vs;
+    uint8_t *flags;
     int *mix_count;
     double *qice;                     // licomqice of the fused icesnow, or NULL
     double area_t;
@@ -869,12 +806,12 @@ struct MemberDev {
     int sf_bx, sf_by;                 // 64 x 4 blocks of the 2-D kernels
     int fd_shape, fd_bx, fd_by;       // prelude column blocks
     int sv_shape, sv_bx, sv_by;       // column-solve blocks
-    int ntx, ntiles;                  // BX x BY k-march tiles
+    FlatGrid ff, fu;                  // limiter flags, update
     int side_vec, side_blocks, side2_blocks;
     int halo_bx;                      // halo blocks per plane (4 km planes + licomqice)
 };
 
-enum { ST_SURF, ST_SSSP, ST_SSSF, ST_FD, ST_WC /* unused */, ST_MARCH, ST_SOLVE, ST_SIDE3, ST_SIDE2, ST_HALO,
+enum { ST_SURF, ST_SSSP, ST_SSSF, ST_FD, ST_FLAGS, ST_MARCH, ST_SOLVE, ST_SIDE3, ST_SIDE2, ST_HALO,
        NSTAGE };
 
 // Member owning global block b of a stage (starts: nm+1 prefix sums).
@@ -919,36 +856,63 @@ __global__ __launch_bounds__(256) void kb_prelude(const MemberDev *M, const int 
                             d.uw, d.vs, l % d.fd_bx, l / d.fd_bx, d.fd_shape);
 }
 
-// Persistent k-march: each workgroup walks the (member, tile, tracer) list.
-__global__ __launch_bounds__(NT, MARCH_BLOCKS) void kb_march(const MemberDev *M, const int *starts, int nm,
-                                                  int total) {
+__device__ __forceinline__ CellsMx member_cells(const MemberDev &d) {
+    CellsMx a;
+    a.at = d.at;
+    a.atb = d.atb;
+    a.stf_n = d.stf_n;
+    a.err_norm2 = d.err_norm2;
+    a.swv = d.swv;
+    a.restore = d.restore;
+    a.akt = d.akt;
+    a.uw = d.uw;
+    a.vs = d.vs;
+    a.ws = d.ws;
+    a.ori = d.ori;
+    a.ax = d.ax;
+    a.ay = d.ay;
+    a.az = d.az;
+    a.dz = d.dz;
+    a.pen = d.pen;
+    a.flags = d.flags;
+    a.flags_out = nullptr;
+    return a;
+}
+
+__global__ __launch_bounds__(256, 4) void kb_flags(const MemberDev *M, const int *starts, int nm, int total) {
+    const int *st_ = starts + ST_FLAGS * (nm + 1);
+    const int it = xcd_item((int)blockIdx.x, (total + 7) / 8);
+    if (it >= total) return;
+    const int m = find_member(st_, nm, it);
+    const MemberDev &d = M[m];
+    const KGrid g = d.g;
+    const FlatGrid fg = d.ff;
+    flags_mx_body(g, d.p.dts, member_cells(d), fg, it - st_[m]);
+}
+
+// Each workgroup walks the (member, run of cells, chunk, tracer) list in
+// strides of the grid (licom_batch_set_march_grid).
+__device__ __forceinline__ void update_items(const MemberDev *M, const int *starts, int nm, int total,
+                                             licom_f2a (*sM)[256]) {
     const int *st_ = starts + ST_MARCH * (nm + 1);
-    for (int it = blockIdx.x; it < total; it += gridDim.x) {
+    const int per = (total + 7) / 8;
+    for (int s = blockIdx.x; s < 8 * per; s += gridDim.x) {
+        const int it = xcd_item(s, per);
+        if (it >= total) continue;
         const int m = find_member(st_, nm, it);
         const MemberDev &d = M[m];
-        const int l = it - st_[m];
-        MarchArgsMx a;
-        a.at = d.at;
-        a.atb = d.atb;
-        a.stf_n = d.stf_n;
-        a.err_norm2 = d.err_norm2;
-        a.swv = d.swv;
-        a.restore = d.restore;
-        a.akt = d.akt;
-        a.uw = d.uw;
-        a.vs = d.vs;
-        a.ws = d.ws;
-        a.ori = d.ori;
-        a.ax = d.ax;
-        a.ay = d.ay;
-        a.az = d.az;
-        a.dz = d.dz;
-        a.pen = d.pen;
-        a.ntx = d.ntx;
-        a.ntiles = d.ntiles;
-        a.tiles_per_xcd = 0;
-        march_body(d.g, d.p, a, l >> 1, l & 1);
+        const KGrid g = d.g;
+        const KPar p = d.p;
+        const FlatGrid fg = d.fu;
+        const CellsMx a = member_cells(d);
+        if (p.hmix == LICOM_HMIX_DEL4) update_mx_body<true>(g, p, a, fg, it - st_[m], sM);
+        else update_mx_body<false>(g, p, a, fg, it - st_[m], sM);
     }
+}
+
+__global__ __launch_bounds__(256, 2) void kb_update(const MemberDev *M, const int *starts, int nm, int total) {
+    __shared__ licom_f2a sM[kSlotsMx][256];
+    update_items(M, starts, nm, total, sM);
 }
 
 template <int KM>
@@ -1018,8 +982,8 @@ __global__ __launch_bounds__(256) void kb_halo(const MemberDev *M, const int *st
 // One launch per step: a grid of co-resident workgroups walks every stage's
 // work list (the same items and bodies as the kb_* launches, so the same
 // bits), with a grid-wide barrier between dependent phases:
-//   surface | SSSNORM partials | SSSNORM total + column prelude | k-march |
-//   column solve | side effects + halo.
+//   surface | SSSNORM partials | SSSNORM total + column prelude | limiter
+//   flags | update | column solve | side effects + halo.
 // The barrier waits are bounded: a workgroup that waits longer than
 // kBarSpins polls (workgroups that are not co-resident, for example with
 // other work on the device) sets the error flag and leaves, every later
@@ -1116,32 +1080,14 @@ __global__ __launch_bounds__(256, 2) void kb_step(const MemberDev *M, const int 
         __syncthreads();
     }
     if (!grid_sync(bar, nblk)) return;
-    for (int it = blockIdx.x; it < T.t[ST_MARCH]; it += G) {
+    for (int it = blockIdx.x; it < T.t[ST_FLAGS]; it += G) {
         int l;
-        const MemberDev &d = member(ST_MARCH, it, l);
-        MarchArgsMx a;
-        a.at = d.at;
-        a.atb = d.atb;
-        a.stf_n = d.stf_n;
-        a.err_norm2 = d.err_norm2;
-        a.swv = d.swv;
-        a.restore = d.restore;
-        a.akt = d.akt;
-        a.uw = d.uw;
-        a.vs = d.vs;
-        a.ws = d.ws;
-        a.ori = d.ori;
-        a.ax = d.ax;
-        a.ay = d.ay;
-        a.az = d.az;
-        a.dz = d.dz;
-        a.pen = d.pen;
-        a.ntx = d.ntx;
-        a.ntiles = d.ntiles;
-        a.tiles_per_xcd = 0;
-        march_body(d.g, d.p, a, l >> 1, l & 1);
-        __syncthreads();
+        const MemberDev &d = member(ST_FLAGS, it, l);
+        flags_mx_body(d.g, d.p.dts, member_cells(d), d.ff, l);
     }
+    if (!grid_sync(bar, nblk)) return;
+    __shared__ licom_f2a sM[kSlotsMx][256];
+    update_items(M, starts, nm, T.t[ST_MARCH], sM);
     if (!grid_sync(bar, nblk)) return;
     for (int it = blockIdx.x; it < T.t[ST_SOLVE]; it += G) {
         int l;
@@ -1298,9 +1244,9 @@ int batch_launch_step(licom_batch *b, int flags) {
     if (b->kmax <= 30) kb_prelude<30><<<grid(ST_FD), 256, 0, st>>>(M, S, nm);
     else if (b->kmax <= 55) kb_prelude<55><<<grid(ST_FD), 256, 0, st>>>(M, S, nm);
     else kb_prelude<LICOM_MAX_KM><<<grid(ST_FD), 256, 0, st>>>(M, S, nm);
-    const int items = b->totals[ST_MARCH];
-    const int mg = b->march_grid > 0 ? std::min(b->march_grid, items) : items;
-    kb_march<<<(unsigned)mg, NT, 0, st>>>(M, S, nm, items);
+    const int nf = b->totals[ST_FLAGS], nu = b->totals[ST_MARCH], gu = (nu + 7) / 8 * 8;
+    kb_flags<<<(unsigned)((nf + 7) / 8 * 8), 256, 0, st>>>(M, S, nm, nf);
+    kb_update<<<(unsigned)(b->march_grid > 0 ? std::min(b->march_grid, gu) : gu), 256, 0, st>>>(M, S, nm, nu);
     if (flags & LICOM_STEP_ICESNOW) {
         if (b->kmax <= 30) kb_solve_ice<30><<<grid(ST_SOLVE), 256, 0, st>>>(M, S, nm, flags);
         else if (b->kmax <= 55) kb_solve_ice<55><<<grid(ST_SOLVE), 256, 0, st>>>(M, S, nm, flags);
@@ -1344,6 +1290,9 @@ extern "C" int licom_batch_create(licom_ctx *const *members, const licom_fields_
     std::vector<MemberDev> hm(n);
     std::vector<int> starts((size_t)NSTAGE * (n + 1), 0);
     int kmax = 0;
+    double cells = 0.0;
+    for (int m = 0; m < n; ++m)
+        if (members[m]) cells += (double)members[m]->n2;
     for (int m = 0; m < n; ++m) {
         licom_ctx *c = members[m];
         const licom_fields_mixed &f = fields[m];
@@ -1430,9 +1379,12 @@ extern "C" int licom_batch_create(licom_ctx *const *members, const licom_fields_
         const dim3 sg = solve_grid(imt, jmt, d.sv_shape);
         d.sv_bx = (int)sg.x;
         d.sv_by = (int)sg.y;
-        d.ntx = (imt - 4 + BX - 1) / BX;
-        d.ntiles = d.ntx * ((jmt - 4 + BY - 1) / BY);
         const size_t n3 = c->n3, n2 = c->n2;
+        d.flags = s.flags;
+        // this member's share of the workgroups that fill the chip
+        const int want = (int)(1024.0 * (double)n2 / cells) + 1;
+        d.ff = flat_grid(imt, (jmt - 1) * imt, km, want);
+        d.fu = flat_grid(2 * imt, (jmt - 2) * imt, km, want);
         d.side_vec = ((reinterpret_cast<uintptr_t>(f.utf) | reinterpret_cast<uintptr_t>(f.vtf)) & 15) == 0 &&
                      n3 % 4 == 0;
         d.side_blocks = (int)(((d.side_vec ? n3 / 4 : n3) + 255) / 256);
@@ -1442,8 +1394,8 @@ extern "C" int licom_batch_create(licom_ctx *const *members, const licom_fields_
                                   d.nblk,
                                   1,
                                   (long)d.fd_bx * d.fd_by,
-                                  0,
-                                  2L * d.ntiles,
+                                  d.ff.total,
+                                  d.fu.total,
                                   (long)d.sv_bx * d.sv_by,
                                   d.side_blocks,
                                   d.side2_blocks,

@@ -3,8 +3,8 @@ C ABI (mixed-precision form).
 
 * :class:`Ensemble` binds ``licom_batch_*``: many members, each a
   :class:`licom_tracer.TracerModel` of its own grid, advance together, one
-  launch per stage and step (the k-march as persistent workgroups over
-  (member, tile, tracer) items); N steps can be captured in a HIP graph and
+  launch per stage and step (the update in strides over its
+  (member, run of cells, tracer) items); N steps can be captured in a HIP graph and
   replayed.
 * :class:`Autotuner` times every launch-shape candidate
   (``licom_autotune_member``) once per (imt, jmt, km) and caches the winner.
