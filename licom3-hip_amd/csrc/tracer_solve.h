@@ -29,51 +29,62 @@ constexpr int SEG = 4;
 // starts is either recomputed by it or belongs to a level that mixing has not
 // touched, so the mask plus on-demand recomputation reproduces its decisions.
 // The two lanes of a column run this together: each holds its own tracer's
-// column X (the state just written, stride n2) and they swap values with
-// __shfl_xor over 32 lanes.  Returns the mixed level range in lo/hi.
+// column X (the state just written, stride n2), the T lane forms the mixed
+// region's density and the S lane the tested level's, and they swap values
+// with __shfl_xor over 32 lanes.  Every step is a link of a serial chain, so
+// what it waits for is kept short: both ends of the region are tested in one
+// step (the lower one decides first), their values are loaded a step ahead,
+// and the coefficients (C, to, so, dzp) come from LDS (solve of 128 x 96 x 30
+// 58 -> 50 us, 225 x 145 x 55 121 -> 103 us, 360 x 218 x 30 with icesnow, half
+// of whose columns mix, 427 -> 377 us).  Returns the mixed level range in
+// lo/hi.
 __device__ __noinline__ void convect_sparse(const double *C, const double *to, const double *so,
                                             const double *dzp, int km, int kcon, uint64_t mask,
                                             int n, double *X, size_t n2, int &lo, int &hi) {
     lo = km;
     hi = -1;
     int lcon = __ffsll((unsigned long long)mask) - 1;
+    auto at = [&](int k) { return X[(size_t)min(max(k, 0), kcon - 1) * n2]; };
+    // the mixed region's density and v's, both at level k
+    auto both = [&](int k, double mix, double v, double &rmix, double &rv) {
+        const double got = __shfl_xor(n == 0 ? v : mix, 32);
+        const double mine = dev::dens(C, km, k, (n == 0 ? mix : got) - to[k], (n == 0 ? got : v) - so[k]);
+        const double other = __shfl_xor(mine, 32);
+        rmix = n == 0 ? mine : other;
+        rv = n == 0 ? other : mine;
+    };
     for (;;) {   // CONV_1
         int lcona = lcon, lconb = lcon + 1;
+        const double x0 = at(lcona - 1), x1 = at(lconb - 1);
+        // the levels below and above the region, and those after them
+        double vb = at(lconb), nb = at(lconb + 1), va = at(lcona - 2), na = at(lcona - 3);
         double dztsum = dzp[lcona - 1] + dzp[lconb - 1];
-        double trasum = X[(size_t)(lcona - 1) * n2] * dzp[lcona - 1] + X[(size_t)(lconb - 1) * n2] * dzp[lconb - 1];
+        double trasum = x0 * dzp[lcona - 1] + x1 * dzp[lconb - 1];
         double tramix = trasum / dztsum;
         for (;;) {   // CONV_2
-            if (lconb != kcon) {
-                const double v = X[(size_t)lconb * n2];
-                const double vo = __shfl_xor(v, 32), mo = __shfl_xor(tramix, 32);
-                const double Tm = n == 0 ? tramix : mo, Sm = n == 0 ? mo : tramix;
-                const double Tv = n == 0 ? v : vo, Sv = n == 0 ? vo : v;
-                const double rl = dev::dens(C, km, lconb, Tm - to[lconb], Sm - so[lconb]);
-                const double ru = dev::dens(C, km, lconb, Tv - to[lconb], Sv - so[lconb]);
-                if (rl > ru) {
-                    lconb = lconb + 1;
-                    dztsum = dztsum + dzp[lconb - 1];
-                    trasum = trasum + v * dzp[lconb - 1];
-                    tramix = trasum / dztsum;
-                    continue;
-                }
+            const bool can_b = lconb != kcon, can_a = lcona > 1;
+            const int kb = can_b ? lconb : lconb - 1;
+            double rmix, rv;
+            both(kb, tramix, vb, rmix, rv);
+            const bool down = can_b && rmix > rv;
+            both(lcona - 1, tramix, va, rmix, rv);
+            const bool up = can_a && rv > rmix;
+            if (down) {
+                dztsum = dztsum + dzp[lconb];
+                trasum = trasum + vb * dzp[lconb];
+                lconb = lconb + 1;
+                vb = nb;
+                nb = at(lconb + 1);
+            } else if (up) {
+                dztsum = dztsum + dzp[lcona - 2];
+                trasum = trasum + va * dzp[lcona - 2];
+                lcona = lcona - 1;
+                va = na;
+                na = at(lcona - 3);
+            } else {
+                break;
             }
-            if (lcona > 1) {
-                const double v = X[(size_t)(lcona - 2) * n2];
-                const double vo = __shfl_xor(v, 32), mo = __shfl_xor(tramix, 32);
-                const double Tm = n == 0 ? tramix : mo, Sm = n == 0 ? mo : tramix;
-                const double Tv = n == 0 ? v : vo, Sv = n == 0 ? vo : v;
-                const double rl = dev::dens(C, km, lcona - 1, Tv - to[lcona - 1], Sv - so[lcona - 1]);
-                const double ru = dev::dens(C, km, lcona - 1, Tm - to[lcona - 1], Sm - so[lcona - 1]);
-                if (rl > ru) {
-                    lcona = lcona - 1;
-                    dztsum = dztsum + dzp[lcona - 1];
-                    trasum = trasum + v * dzp[lcona - 1];
-                    tramix = trasum / dztsum;
-                    continue;
-                }
-            }
-            break;
+            tramix = trasum / dztsum;
         }
         for (int l = lcona - 1; l < lconb; ++l) X[(size_t)l * n2] = tramix;
         lo = min(lo, lcona - 1);
@@ -119,12 +130,13 @@ __device__ __forceinline__ void solve_body(const KGrid &g, const KPar &p, int fl
     // be scalar loads, and every vector load's wait would also wait for the
     // stores issued before it (one vmcnt covers both on gfx9).
     __shared__ double sZP[LICOM_MAX_KM], sZT[LICOM_MAX_KM], sTO[LICOM_MAX_KM], sSO[LICOM_MAX_KM];
-    __shared__ double sC[9 * LICOM_MAX_KM];
+    __shared__ double sC[9 * LICOM_MAX_KM], sDZ[LICOM_MAX_KM];
     for (int r = t; r < km; r += 256) {
         sZP[r] = g.odzp[r];
         sZT[r] = g.odzt[r];
         sTO[r] = g.to[r];
         sSO[r] = g.so[r];
+        sDZ[r] = g.dzp[r];
     }
     for (int r = t; r < 9 * km; r += 256) sC[r] = g.eosc[r];
     __syncthreads();
@@ -350,7 +362,7 @@ __device__ __forceinline__ void solve_body(const KGrid &g, const KPar &p, int fl
                     if (dt_diff) __builtin_nontemporal_store((DG)v, &dt_diff[c]);
                     if (tend) __builtin_nontemporal_store((DG)tn, &tend[c]);
                     if (conv && dt_conv) __builtin_nontemporal_store((DG)0.0, &dt_conv[c]);
-                    __builtin_nontemporal_store(xs, &Tb[(size_t)k * n2 + q]);
+                    Tb[(size_t)k * n2 + q] = xs;     // the mixing reads it again
                     __builtin_nontemporal_store(x, &Bb[(size_t)k * n2 + q]);
                 }
                 if (conv) {
@@ -382,15 +394,27 @@ __device__ __forceinline__ void solve_body(const KGrid &g, const KPar &p, int fl
         if (conv && act && mask != 0) {
             if (n == 0) atomicAdd(mix_count, 1);
             int lo, hi;
-            convect_sparse(g.eosc, g.to, g.so, g.dzp, km, kz, mask, n, TT, n2, lo, hi);
-            for (int l = lo; l <= hi; ++l) {
-                const size_t c = (size_t)l * n2;
-                const double y = TT[c], b = BB[c];
-                if (y != b) {
-                    const double dc = (y - b) / dts * 1.0;
-                    if (dt_conv) dt_conv[n * n3 + q + c] = (DG)dc;
-                    if (tend) tend[n * n3 + q + c] = (DG)((double)tend[n * n3 + q + c] + dc);
-                    BB[c] = y;
+            convect_sparse(sC, sTO, sSO, sDZ, km, kz, mask, n, TT, n2, lo, hi);
+            // four levels' loads wait together
+            constexpr int W = 4;
+            for (int l0 = lo; l0 <= hi; l0 += W) {
+                double y[W], b[W], td[W];
+#pragma unroll
+                for (int r = 0; r < W; ++r) {
+                    const size_t c = (size_t)min(l0 + r, hi) * n2;
+                    y[r] = TT[c];
+                    b[r] = BB[c];
+                    td[r] = tend ? (double)tend[n * n3 + q + c] : 0.0;
+                }
+#pragma unroll
+                for (int r = 0; r < W; ++r) {
+                    const size_t c = (size_t)(l0 + r) * n2;
+                    if (l0 + r <= hi && y[r] != b[r]) {
+                        const double dc = (y[r] - b[r]) / dts * 1.0;
+                        if (dt_conv) dt_conv[n * n3 + q + c] = (DG)dc;
+                        if (tend) tend[n * n3 + q + c] = (DG)(td[r] + dc);
+                        BB[c] = y[r];
+                    }
                 }
             }
         }
@@ -404,7 +428,7 @@ __device__ __forceinline__ void solve_body(const KGrid &g, const KPar &p, int fl
         int lo = km, hi = -1;
         if (mask != 0) {   // the same in both lanes of the pair
             if (n == 0) atomicAdd(mix_count, 1);
-            convect_sparse(g.eosc, g.to, g.so, g.dzp, km, kz, mask, n, TT, n2, lo, hi);
+            convect_sparse(sC, sTO, sSO, sDZ, km, kz, mask, n, TT, n2, lo, hi);
         }
         for (int l = 0; l < km; ++l) {
             if ((l < lo || l > hi) && !((icemask >> l) & 1ull)) continue;
