@@ -294,10 +294,16 @@ __device__ __forceinline__ double viv_of(const Column &C, const double *__restri
     return C.v01 ? (((C.vone >> k) & 1ull) ? 1.0 : 0.0) : viv[c];
 }
 
+// Levels of the in-place updates whose loads are issued together: the compiler
+// must assume that a level's stores alias the next one's loads, so one level
+// at a time a column waited for memory 55 times (360 x 231 x 55, a leapfrog
+// step with the wave-sized blocks: 902 -> 783 us).
+constexpr int kGroup = 8;
+
 // bclinc4_cu (bclinc.cpp:266-379) or bclinc81_cu + bclinc82_cu (:670-726)
 template <bool EULER>
 __global__ __launch_bounds__(256) void k_bcl_b(BGrid g, licom_bclinc_fields f) {
-    const int i = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * 4 + threadIdx.y;
+    const int i = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * blockDim.y + threadIdx.y;
     const int imt = g.imt, jmt = g.jmt, km = g.km;
     if (i >= imt || j >= jmt) return;
     const size_t n2 = g.n2, q = (size_t)j * imt + i;
@@ -327,13 +333,30 @@ __global__ __launch_bounds__(256) void k_bcl_b(BGrid g, licom_bclinc_fields f) {
     const bool in2 = interior2(g, j, i);
     const double vb = f.vb[q];
 #pragma unroll
-    for (int k = 0; k < LICOM_MAX_KM; ++k) {
-        if (k < km) {
-            const size_t c = (size_t)k * n2 + q;
-            const double w = (C.x[k] - C.work + vb) * viv_of(C, f.viv, c, k);
-            f.vp[c] = g.afc2 * f.v[c] + g.afc1 * (f.vp[c] + w);
-            f.v[c] = w;
-            f.wka[c] = in2 ? f.up[c] + f.dlu[c] * g.dtc2 : w;
+    for (int k0 = 0; k0 < LICOM_MAX_KM; k0 += kGroup) {
+        double v[kGroup] = {}, vp[kGroup] = {}, up[kGroup] = {}, dlu[kGroup] = {};
+#pragma unroll
+        for (int r = 0; r < kGroup; ++r) {
+            if (k0 + r < km) {
+                const size_t c = (size_t)(k0 + r) * n2 + q;
+                v[r] = f.v[c];
+                vp[r] = f.vp[c];
+                if (in2) {
+                    up[r] = f.up[c];
+                    dlu[r] = f.dlu[c];
+                }
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < kGroup; ++r) {
+            const int k = k0 + r;
+            if (k < km) {
+                const size_t c = (size_t)k * n2 + q;
+                const double w = (C.x[k] - C.work + vb) * viv_of(C, f.viv, c, k);
+                f.vp[c] = g.afc2 * v[r] + g.afc1 * (vp[r] + w);
+                f.v[c] = w;
+                f.wka[c] = in2 ? up[r] + dlu[r] * g.dtc2 : w;
+            }
         }
     }
     if (!in2) return;
@@ -343,7 +366,7 @@ __global__ __launch_bounds__(256) void k_bcl_b(BGrid g, licom_bclinc_fields f) {
 
 // bclinc5_cu (bclinc.cpp:381-416)
 __global__ __launch_bounds__(256) void k_bcl_c(BGrid g, licom_bclinc_fields f) {
-    const int i = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * 4 + threadIdx.y;
+    const int i = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * blockDim.y + threadIdx.y;
     const int imt = g.imt, jmt = g.jmt, km = g.km;
     if (i >= imt || j >= jmt) return;
     const size_t n2 = g.n2, q = (size_t)j * imt + i;
@@ -351,14 +374,30 @@ __global__ __launch_bounds__(256) void k_bcl_c(BGrid g, licom_bclinc_fields f) {
     Column C;
     load_column(g, f.wka, f.viv, q, ohbu, C);
 #pragma unroll
-    for (int k = 0; k < LICOM_MAX_KM; ++k) {
-        if (k < km) {
-            const size_t c = (size_t)k * n2 + q;
-            const double w = (C.x[k] - C.work + ub) * viv_of(C, f.viv, c, k);
-            f.up[c] = g.afc2 * f.u[c] + g.afc1 * (f.up[c] + w);
-            f.u[c] = w;
-            f.utf[c] += w;
-            f.vtf[c] += f.v[c];
+    for (int k0 = 0; k0 < LICOM_MAX_KM; k0 += kGroup) {
+        double u[kGroup] = {}, up[kGroup] = {}, v[kGroup] = {}, utf[kGroup] = {}, vtf[kGroup] = {};
+#pragma unroll
+        for (int r = 0; r < kGroup; ++r) {
+            if (k0 + r < km) {
+                const size_t c = (size_t)(k0 + r) * n2 + q;
+                u[r] = f.u[c];
+                up[r] = f.up[c];
+                v[r] = f.v[c];
+                utf[r] = f.utf[c];
+                vtf[r] = f.vtf[c];
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < kGroup; ++r) {
+            const int k = k0 + r;
+            if (k < km) {
+                const size_t c = (size_t)k * n2 + q;
+                const double w = (C.x[k] - C.work + ub) * viv_of(C, f.viv, c, k);
+                f.up[c] = g.afc2 * u[r] + g.afc1 * (up[r] + w);
+                f.u[c] = w;
+                f.utf[c] = utf[r] + w;
+                f.vtf[c] = vtf[r] + v[r];
+            }
         }
     }
 }
@@ -492,6 +531,9 @@ int licom_bclinc_stage(licom_bclinc *b, const licom_bclinc_fields *f, int isc, i
         }
     const BGrid &g = b->g;
     const dim3 blk(64, 4), grd((g.imt + 63) / 64, (g.jmt + 3) / 4);
+    // columns that share nothing go out a wave at a time, so that the CUs'
+    // shares differ by a wave and not by four
+    const dim3 wave(64, 1), rows((g.imt + 63) / 64, g.jmt);
     const bool euler = isc < 1;
     if (int rc = hip_status(hipEventRecord(b->ev0, b->stream), "hipEventRecord")) return rc;
     if (stage == 0) {
@@ -504,12 +546,12 @@ int licom_bclinc_stage(licom_bclinc *b, const licom_bclinc_fields *f, int isc, i
         if (int rc = hip_status(hipGetLastError(), "k_bcl_a launch")) return rc;
     } else if (stage == 1) {
         if (euler)
-            k_bcl_b<true><<<grd, blk, 0, b->stream>>>(g, *f);
+            k_bcl_b<true><<<rows, wave, 0, b->stream>>>(g, *f);
         else
-            k_bcl_b<false><<<grd, blk, 0, b->stream>>>(g, *f);
+            k_bcl_b<false><<<rows, wave, 0, b->stream>>>(g, *f);
         if (int rc = hip_status(hipGetLastError(), "k_bcl_b launch")) return rc;
     } else {
-        k_bcl_c<<<grd, blk, 0, b->stream>>>(g, *f);
+        k_bcl_c<<<rows, wave, 0, b->stream>>>(g, *f);
         if (int rc = hip_status(hipGetLastError(), "k_bcl_c launch")) return rc;
     }
     if (int rc = hip_status(hipEventRecord(b->ev1, b->stream), "hipEventRecord")) return rc;
