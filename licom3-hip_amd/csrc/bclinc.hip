@@ -45,6 +45,13 @@ __device__ __forceinline__ bool interior2(const BGrid &g, int j, int i) {
     return i >= 2 && i < g.imt - 2 && j >= 2 && j < g.jmt - 2;
 }
 
+// Levels of a column whose loads are issued together: the compiler must assume
+// that a level's stores alias the next one's loads, so one level at a time a
+// column waited for memory 55 times (360 x 231 x 55, a leapfrog step: 902 us;
+// 783 with the updates of k_bcl_b/c in groups and wave-sized blocks, 662 with
+// the solve's sweeps in groups as well).
+constexpr int kGroup = 8;
+
 // The implicit vertical viscosity of one U column (bclinc3_cu :197-259,
 // bclinc4_cu :301-374, bclinc71_cu :498-576, bclinc72_cu :589-667): x holds
 // the explicit update at levels 0..kz-1 and receives the solution there.
@@ -54,41 +61,69 @@ __device__ void column_solve(const BGrid &g, const double *__restrict__ akmu, co
     const double *odzt = g.odzt, *odzp = g.odzp;
     // elimination from the bottom: e8(k), f8(k) from level k+1's
     double en = 0.0, fn = 0.0;   // e8(kz) = f8(kz) = 0
-    for (int k = kz - 1; k >= 0; --k) {
-        const size_t c = (size_t)k * n2 + q;
-        double a8, b8, c8, d8;
-        if (k == kz - 1) {
-            // bottom condition; a8 as the level above it set it
-            a8 = k >= 1 ? akmu[c - n2] * odzt[k] * odzp[k] * dt * 0.5 : odzp[0] * dt * 0.5;
-            b8 = 1.0 + a8;
-            c8 = odzp[k] * dt * 0.5;
-            d8 = x[c] - bbc * odzp[k] * dt * 0.5;
-        } else if (k == 0) {
-            a8 = odzp[0] * dt * 0.5;
-            c8 = akmu[c] * odzt[1] * odzp[0] * dt * 0.5;
-            b8 = 1.0 + c8;
-            d8 = x[c];
-        } else {
-            a8 = akmu[c - n2] * odzt[k] * odzp[k] * dt * 0.5;
-            c8 = akmu[c] * odzt[k + 1] * odzp[k] * dt * 0.5;
-            b8 = 1.0 + a8 + c8;
-            d8 = x[c];
+    double ak = 0.0;             // akmu at level k, loaded for level k + 1
+    for (int kt = kz - 1; kt >= 0; kt -= kGroup) {
+        double d[kGroup] = {}, am[kGroup] = {};
+#pragma unroll
+        for (int r = 0; r < kGroup; ++r) {
+            const int k = kt - r;
+            if (k >= 0) d[r] = x[(size_t)k * n2 + q];
+            if (k >= 1) am[r] = akmu[(size_t)(k - 1) * n2 + q];
         }
-        const double g0 = 1.0 / (b8 - c8 * en);
-        const double e = a8 * g0;
-        const double fv = (d8 + c8 * fn) * g0;
-        g.e8[c] = e;
-        g.f8[c] = fv;
-        en = e;
-        fn = fv;
+#pragma unroll
+        for (int r = 0; r < kGroup; ++r) {
+            const int k = kt - r;
+            if (k < 0) continue;
+            const size_t c = (size_t)k * n2 + q;
+            double a8, b8, c8, d8;
+            if (k == kz - 1) {
+                // bottom condition; a8 as the level above it set it
+                a8 = k >= 1 ? am[r] * odzt[k] * odzp[k] * dt * 0.5 : odzp[0] * dt * 0.5;
+                b8 = 1.0 + a8;
+                c8 = odzp[k] * dt * 0.5;
+                d8 = d[r] - bbc * odzp[k] * dt * 0.5;
+            } else if (k == 0) {
+                a8 = odzp[0] * dt * 0.5;
+                c8 = ak * odzt[1] * odzp[0] * dt * 0.5;
+                b8 = 1.0 + c8;
+                d8 = d[r];
+            } else {
+                a8 = am[r] * odzt[k] * odzp[k] * dt * 0.5;
+                c8 = ak * odzt[k + 1] * odzp[k] * dt * 0.5;
+                b8 = 1.0 + a8 + c8;
+                d8 = d[r];
+            }
+            const double g0 = 1.0 / (b8 - c8 * en);
+            const double e = a8 * g0;
+            const double fv = (d8 + c8 * fn) * g0;
+            g.e8[c] = e;
+            g.f8[c] = fv;
+            en = e;
+            fn = fv;
+            ak = am[r];
+        }
     }
     // substitution from the surface
     double prev = sbc;
-    for (int k = 0; k < kz; ++k) {
-        const size_t c = (size_t)k * n2 + q;
-        const double v = (g.e8[c] * prev + g.f8[c]) * viv[c];
-        x[c] = v;
-        prev = v;
+    for (int kt = 0; kt < kz; kt += kGroup) {
+        double e[kGroup] = {}, fv[kGroup] = {}, vv[kGroup] = {};
+#pragma unroll
+        for (int r = 0; r < kGroup; ++r) {
+            if (kt + r < kz) {
+                const size_t c = (size_t)(kt + r) * n2 + q;
+                e[r] = g.e8[c];
+                fv[r] = g.f8[c];
+                vv[r] = viv[c];
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < kGroup; ++r) {
+            if (kt + r < kz) {
+                const double v = (e[r] * prev + fv[r]) * vv[r];
+                x[(size_t)(kt + r) * n2 + q] = v;
+                prev = v;
+            }
+        }
     }
 }
 
@@ -293,12 +328,6 @@ __device__ __forceinline__ void load_column(const BGrid &g, const double *__rest
 __device__ __forceinline__ double viv_of(const Column &C, const double *__restrict__ viv, size_t c, int k) {
     return C.v01 ? (((C.vone >> k) & 1ull) ? 1.0 : 0.0) : viv[c];
 }
-
-// Levels of the in-place updates whose loads are issued together: the compiler
-// must assume that a level's stores alias the next one's loads, so one level
-// at a time a column waited for memory 55 times (360 x 231 x 55, a leapfrog
-// step with the wave-sized blocks: 902 -> 783 us).
-constexpr int kGroup = 8;
 
 // bclinc4_cu (bclinc.cpp:266-379) or bclinc81_cu + bclinc82_cu (:670-726)
 template <bool EULER>
