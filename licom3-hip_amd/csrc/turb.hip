@@ -45,6 +45,7 @@
 
 #include "licom_turb.h"
 #include "tracer_internal.h"
+#include "turb_shape.h"
 
 namespace licom {
 namespace {
@@ -52,9 +53,6 @@ namespace {
 constexpr int MT = LICOM_TURB_MT, MT0 = LICOM_TURB_MT0, NTH = LICOM_TURB_NTH;
 constexpr int W2 = 2 * MT + 1;      // entries of a 1-D table
 constexpr int NB = 4 * NTH + 1;     // entries of a background table
-// One wave, so that the CUs' shares differ by a wave and not by four
-// (360 x 218 x 30: 560 -> 507 us).
-constexpr int TPB = 64;
 
 struct alignas(32) Q4 {   // {slq2, sm, sh, ss} or {amtaun2, sm, sh, ss}
     double v[4];
@@ -199,16 +197,16 @@ __device__ double eplat_den() {
     return f30 * acosh(an0 / f30);
 }
 
-__global__ __launch_bounds__(TPB) void k_turb(TurbArgs a) {
+__global__ __launch_bounds__(256) void k_turb(TurbArgs a) {
     __shared__ double sZ[LICOM_MAX_KM + 1], sD[LICOM_MAX_KM];
     const int km = a.km;
-    for (int r = threadIdx.x; r <= km; r += TPB) {
+    for (int r = threadIdx.x; r <= km; r += blockDim.x) {
         sZ[r] = a.zkp[r];
         if (r < km) sD[r] = a.dzp[r];
     }
     __syncthreads();
     const size_t n2 = a.n2;
-    const size_t q = (size_t)blockIdx.x * TPB + threadIdx.x;
+    const size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= n2) return;
     const licom_turb_fields &F = a.f;
     const int i = (int)(q % (size_t)a.imt), j = (int)(q / (size_t)a.imt);
@@ -654,9 +652,9 @@ int licom_turb_run(licom_turb *t, const licom_turb_fields *f) {
             return LICOM_EINVAL;
         }
     t->args.f = *f;
-    const unsigned blocks = (unsigned)((t->n2 + TPB - 1) / TPB);
+    const unsigned lanes = (unsigned)turb_lanes(t->n2), blocks = (unsigned)((t->n2 + lanes - 1) / lanes);
     if (int rc = hip_status(hipEventRecord(t->ev0, t->stream), "hipEventRecord")) return rc;
-    hipLaunchKernelGGL(k_turb, dim3(blocks), dim3(TPB), 0, t->stream, t->args);
+    hipLaunchKernelGGL(k_turb, dim3(blocks), dim3(lanes), 0, t->stream, t->args);
     if (int rc = hip_status(hipGetLastError(), "k_turb launch")) return rc;
     if (int rc = hip_status(hipEventRecord(t->ev1, t->stream), "hipEventRecord")) return rc;
     t->ran = true;
