@@ -187,12 +187,13 @@ def ensemble_cases(n=64, seed0=4000, shape_seed=4999):
 def member_bytes(nx, ny, km):
     """HBM held by one resident mixed-precision member: FP64 at/atb, FP32
     akt/velocities/ws and diagnostics, the context's scratch (ori and the face
-    velocities in FP64-sized buffers) and the 2-D fields."""
+    velocities in FP64-sized buffers, a byte of limiter flags per tracer cell)
+    and the 2-D fields."""
     n2 = (nx + 4) * (ny + 4)
     n3 = n2 * km
     state = 8 * (2 * n3 + 2 * (n3 + n2)) + 4 * (2 * n3 + 4 * n3 + (n3 + n2))
     diag = 4 * (14 * n3 + n3) + 8 * 2 * n2
-    scratch = 8 * (2 * n3 + 2 * n3) + 8 * 12 * n2
+    scratch = 8 * (2 * n3 + 2 * n3) + 2 * n3 + 8 * 12 * n2
     return state + diag + scratch + 8 * 16 * n2
 
 
