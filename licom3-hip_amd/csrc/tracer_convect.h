@@ -1,6 +1,6 @@
 // tracer_convect.h -- convadj of one column, as the column solve runs it.
-// On its own, so that it also compiles for the host (oracle/convect_driver.cpp
-// runs its two lanes as threads, with bounds checks).
+// On its own, so that it also compiles for the host, where a test runs its two
+// lanes as threads, with bounds checks.
 #pragma once
 #include <hip/hip_runtime.h>
 
