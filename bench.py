@@ -39,8 +39,10 @@ def kernel_algorithmic_bytes(name, case, variant="fp64"):
             # utf vtf utl vtl (f32) -> u_wface v_sface ws (f32); the divergence
             # profile stays in registers
             "k_prelude": 4 * 4 + 4 * 3,
-            # at atb (f64 x2) akt (f32 x2) faces ws (f32) -> ori (f64 x2), ax ay az dz (f32 x2), pen
-            "k_march": 8 * 4 + 4 * 2 + 4 * 3 + 8 * 2 + 4 * 8 + 4,
+            # at (f64 x2) faces ws (f32) -> flags (1 B x2)
+            "k_flags": 8 * 2 + 4 * 3 + 2,
+            # at atb (f64 x2) akt (f32 x2) faces ws (f32) flags -> ori (f64 x2), ax ay az dz (f32 x2), pen
+            "k_update": 8 * 4 + 4 * 2 + 4 * 3 + 2 + 8 * 2 + 4 * 8 + 4,
             # ori at (f64 x2) akt (f32 x2) -> at atb (f64 x2) tend dt_diff dt_conv (f32 x2)
             "k_solve": 8 * 4 + 4 * 2 + 8 * 4 + 4 * 6,
             # utf vtf (f32) read and written
@@ -52,8 +54,10 @@ def kernel_algorithmic_bytes(name, case, variant="fp64"):
         # utf vtf utl vtl -> u_wface v_sface ws; the divergence profile stays
         # in registers
         "k_prelude": 8 * 4 + 8 * 3,
-        # at atb akt (x2) u_wface v_sface ws -> ori ax ay az dz (x2), penetrate
-        "k_march": 8 * (6 + 3) + 8 * (10 + 1),
+        # at (x2) u_wface v_sface ws -> flags (1 B x2)
+        "k_flags": 8 * (2 + 3) + 2,
+        # at atb akt (x2) u_wface v_sface ws flags -> ori ax ay az dz (x2), penetrate
+        "k_update": 8 * (6 + 3) + 2 + 8 * (10 + 1),
         # ori akt at (x2) -> at atb tend dt_diff dt_conv (x2)
         "k_solve": 8 * 6 + 8 * 10,
         # utf vtf read and written
@@ -780,7 +784,7 @@ def run_ensemble(args, torch, lt, le):
             "ms_per_step": 1000.0 * dt / (24 * reps), "graph_steps": 24, "replays": reps,
             "launches_per_step": 1, "persistent_workgroups": pgrid,
             "per_stage_launches": {"ms_per_step": 1000.0 * dt_stages / (24 * reps),
-                                   "value": ups * 24 * reps / dt_stages, "launches_per_step": 9},
+                                   "value": ups * 24 * reps / dt_stages, "launches_per_step": 10},
             "step_roofline": {"bytes_per_update": sb, "achieved": round(sb * value / 1e9, 1),
                               "peak": HBM_PEAK_GBS, "unit": "GB/s",
                               "frac": round(sb * value / 1e9 / HBM_PEAK_GBS, 4)},

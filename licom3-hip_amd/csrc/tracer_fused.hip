@@ -190,14 +190,13 @@ __global__ __launch_bounds__(256) void k_prelude_col(KGrid g, KPar p, const doub
 // --------------------------------------------------- limiter flags and update
 // Replaces a march of 16 x 12 tiles whose planes a fourth wave staged in LDS
 // (two barriers a level, two workgroups per CU: bound by the latency of its
-// level loop, 7.03 ms at 1800 x 1151 x 55, 71 us at 128 x 96 x 30; now 6.5 ms
-// and 31 us, k_flags bound by its ~200 FP64 instructions a cell and k_update
-// by its 11 + 8 planes of HBM traffic, 4.2 TB/s).
-// Neither kernel carries anything from one level to the next but values it
-// has already loaded, so a column is cut into chunks of levels and every
-// (chunk, run of cells, tracer) is a workgroup of its own.
-//  Runs of cells and
-// chunks: tracer_cells.h.
+// level loop, 7.03 ms at 1800 x 1151 x 55, 71 us at 128 x 96 x 30; now 6.65 ms
+// and 32 us, k_flags bound by its ~200 FP64 instructions a cell and k_update
+// by its 11 + 8 planes of HBM traffic, 4.2 TB/s; at 3600 x 2302 x 55 the pair
+// takes what the march did, 27 ms).  Neither kernel carries anything from one
+// level to the next but values it has already loaded, so a column is cut into
+// chunks of levels and every (chunk, run of cells, tracer) is a workgroup of
+// its own.  Runs of cells and chunks: tracer_cells.h.
 
 // tspas predictor and limiter flag (advection_tracer_2, tracer.cpp:311-545),
 // one byte per cell, of every cell off the outermost rows and columns (the
@@ -308,6 +307,10 @@ struct UpdateArgs {
 // ax/ay/az/dz/penetrate diagnostics.  The biharmonic operator's first pass is
 // formed again for the rows on both sides of the lane's own (two more loads
 // of atb a level, where its 16 bytes a cell would be written and read back).
+// Waves per SIMD: del4 two (its 19 slots of metrics leave LDS for two
+// workgroups).  del2 three, with 16 registers a lane spilled; at two nothing
+// spills and it takes as long (4.78 against 4.81 ms at 1800 x 1151 x 55, 112
+// against 114 us at 360 x 218 x 30, 21 us both at 128 x 96 x 30).
 template <int ADV, bool DEL4>
 __global__ __launch_bounds__(256, DEL4 ? 2 : 3) void k_update(KGrid g, KPar p, const double *__restrict__ at,
                                                    const double *__restrict__ atb, const double *__restrict__ akt,
@@ -600,11 +603,12 @@ template <int ADV>
 void launch_update(licom_ctx *ctx, const licom_fields *f, const licom_diag *d, const Scratch &s) {
     const KGrid &g = ctx->g;
     hipStream_t st = ctx->stream;
-    Timer t(ctx, "k_march");     // one name for both, as in the mixed form
     if constexpr (ADV == LICOM_ADV_TSPAS) {
+        Timer t(ctx, "k_flags");
         const FlatGrid fg = flat_grid(g.imt, (g.jmt - 1) * g.imt, g.km);
         k_flags<<<8 * fg.per, 256, 0, st>>>(g, ctx->kp.dts, f->at, s.uw, s.vs, f->ws, s.flags, g.odzp, g.odzt, fg);
     }
+    Timer t(ctx, "k_update");
     UpdateArgs a{};
     a.stf_n = s.stf_n;
     a.err_norm2 = s.err_norm2;

@@ -736,7 +736,6 @@ int launch_step_mixed(licom_ctx *ctx, const licom_fields_mixed *f, const licom_d
     if (int rc = launch_surface(ctx, &f64, &d64, ctx->s)) return rc;
     launch_column_mx(ctx, f, d, flags, true);
     {
-        Timer t(ctx, "k_march");
         CellsMx a{};
         a.at = f->at;
         a.atb = f->atb;
@@ -757,7 +756,11 @@ int launch_step_mixed(licom_ctx *ctx, const licom_fields_mixed *f, const licom_d
         a.flags = s.flags;
         a.flags_out = ctx->flags_out;
         const FlatGrid ff = flat_grid(g.imt, (g.jmt - 1) * g.imt, g.km);
-        k_flags_mx<<<8 * ff.per, 256, 0, st>>>(g, ctx->kp.dts, a, ff);
+        {
+            Timer t(ctx, "k_flags");
+            k_flags_mx<<<8 * ff.per, 256, 0, st>>>(g, ctx->kp.dts, a, ff);
+        }
+        Timer t(ctx, "k_update");
         const FlatGrid fu = flat_grid(2 * g.imt, (g.jmt - 2) * g.imt, g.km);
         if (ctx->kp.hmix == LICOM_HMIX_DEL4) k_update_mx<true><<<8 * fu.per, 256, 0, st>>>(g, ctx->kp, a, fu);
         else k_update_mx<false><<<8 * fu.per, 256, 0, st>>>(g, ctx->kp, a, fu);
@@ -1303,7 +1306,8 @@ extern "C" int licom_batch_create(licom_ctx *const *members, const licom_fields_
         }
         const uintptr_t al = reinterpret_cast<uintptr_t>(f.at) | reinterpret_cast<uintptr_t>(f.atb);
         if (c->imt % 2 != 0 || (al & 15) != 0) {
-            set_error("licom_batch_create: member %d needs an even imt and 16-byte aligned at/atb", m);
+            set_error("licom_batch_create: member %d needs an even imt and 16-byte aligned at/atb (the mixed "
+                      "form's limits)", m);
             return LICOM_ENOTSUP;
         }
         if (c->p.boundary_restore == 1 && !f.restore) {
