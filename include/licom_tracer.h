@@ -171,10 +171,12 @@ int licom_tracer_step(licom_ctx *ctx, const licom_fields *f,
  * scratch in a static device array of 170 MiB per device instead of the
  * context's allocation.  Grids whose scratch without the limiter flags,
  * 32*imt*jmt*km + 44*imt*jmt bytes, exceeds 160 MiB (e.g. larger than
- * 360 x 218 x 55) get LICOM_EINVAL; LICOM_STEP_STAGED, an odd imt, arrays
- * not 16-byte aligned and ICESNOW with VTL_SCRATCH get LICOM_ENOTSUP.  Every call on a device shares that device's array:
- * calls that overlap on one device race.  No counterpart in the reference
- * (tracer.cpp:1701 allocates its scratch once at start-up, cuda_init.cpp). */
+ * 360 x 218 x 55) get LICOM_EINVAL; LICOM_STEP_STAGED, ICESNOW with
+ * VTL_SCRATCH, an odd imt and at, atb, ws or akt not 16-byte aligned get
+ * LICOM_ENOTSUP (licom_tracer_step takes any imt and alignment).  Every call
+ * on a device shares that device's array: calls that overlap on one device
+ * race.  No counterpart in the reference (tracer.cpp:1701 allocates its
+ * scratch once at start-up, cuda_init.cpp). */
 int licom_tracer_step_noalloc(licom_ctx *ctx, const licom_fields *f,
                               const licom_diag *d, int flags);
 
@@ -208,8 +210,8 @@ typedef struct licom_diag_mixed {
 } licom_diag_mixed;
 
 /* The step in the mixed-precision form; flags as licom_tracer_step except
- * LICOM_STEP_VTL_SCRATCH and LICOM_STEP_STAGED (LICOM_ENOTSUP).  Needs an
- * even imt and 16-byte aligned at/atb; tspas only (other schemes:
+ * LICOM_STEP_VTL_SCRATCH and LICOM_STEP_STAGED (LICOM_ENOTSUP).  Takes an
+ * even imt and 16-byte aligned at/atb, and tspas, only (otherwise
  * LICOM_ENOTSUP, as for batches). */
 int licom_tracer_step_mixed(licom_ctx *ctx, const licom_fields_mixed *f,
                             const licom_diag_mixed *d, int flags);
@@ -247,7 +249,8 @@ int licom_batch_set_march_grid(licom_batch *b, int workgroups);
  * grid of co-resident workgroups (occupancy x CUs) walks every stage's work
  * list, with a grid-wide barrier between dependent phases (surface |
  * SSSNORM partials | SSSNORM total + prelude | limiter flags | update |
- * solve | side effects + halo).  Same results bit for bit as the default of one launch per stage.
+ * solve | side effects + halo).  Same results bit for bit as the default of
+ * one launch per stage.
  * The barrier waits are bounded: if the workgroups cannot all be resident
  * (other work sharing the device) a wait times out after about a second and
  * licom_batch_sync returns LICOM_EHIP (the members' state is then
@@ -357,10 +360,11 @@ size_t licom_scratch_bytes(const licom_ctx *ctx);
 int licom_last_mix_count(licom_ctx *ctx, int *count);
 
 /* Diagnostic output of the tspas limiter's decisions: every step of the
- * fused FP64 path and of the mixed form writes, for each physical cell of
- * each tracer, 1 where the cell's predictor left its local bounds (its faces
- * take the upwind flux, advection_tracer_3, tracer.cpp:549-921) and 0
- * elsewhere, into flags ([2][km][jmt][imt] bytes, device); NULL stops it.
+ * FP64 form (LICOM_STEP_STAGED apart) and of the mixed form writes, for each
+ * physical cell of each tracer, 1 where the cell's predictor left its local
+ * bounds (its faces take the upwind flux, advection_tracer_3,
+ * tracer.cpp:549-921) and 0 elsewhere, into flags ([2][km][jmt][imt] bytes,
+ * device); NULL stops it.
  * Used to count the decisions the mixed form takes differently from FP64.
  * No reference counterpart (the reference keeps them in its at00/atmax/atmin
  * scratch). */

@@ -187,8 +187,8 @@ int check_fields(const licom_fields *f) {
 }  // namespace
 
 // Checks the arguments of an FP64 step and settles its path: STAGED is added
-// where the fused kernels cannot run the layout, and split is set when
-// convadj must run as a separate pass after the step.
+// for icesnow with VTL_SCRATCH (the fused kernels run every layout), and split
+// is set when convadj must run as a separate pass after the step.
 int plan_step(licom_ctx *c, const licom_fields *f, int &flags, bool &split, const char *who) {
     split = false;
     if (!c || !f) {

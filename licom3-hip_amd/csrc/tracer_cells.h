@@ -27,9 +27,10 @@ struct FlatGrid {
 
 // Whole columns, where those give the 256 CUs four workgroups each (smaller
 // chunks read the levels around them again: at 1800 x 1151 x 55 chunks of 55,
-// 28, 14 and 7 levels took 7.3, 7.7, 8.1 and 8.7 ms for both kernels), and
-// otherwise as many chunks as that takes (want: its share of the 1024
-// workgroups), of two levels at least.
+// 28, 14 and 7 levels take 6.65, 6.69, 6.79 and 7.16 ms for both FP64 kernels),
+// and otherwise as many chunks as that takes (want: its share of the 1024
+// workgroups), of two levels at least.  A plane has five rows or more, so it
+// is never without cells.
 inline FlatGrid flat_grid(int first, int last, int km, int want = 1024) {
     const int nb = (last - first + 4 * kWaveCells - 1) / (4 * kWaveCells);
     int nch = std::max((want + 2 * nb - 1) / (2 * nb), 1);
@@ -40,9 +41,9 @@ inline FlatGrid flat_grid(int first, int last, int km, int want = 1024) {
 }
 
 // Block -> (tracer, chunk, block of the plane): the two tracers of one place,
-// then its chunks, run next to each other, and the hardware's round-robin deal of blocks to
-// the eight XCDs is undone, so that each XCD's L2 sees a run of neighbouring
-// blocks, whose rows and face velocities they share.
+// then its chunks, run next to each other, and the hardware's round-robin deal
+// of blocks to the eight XCDs is undone, so that each XCD's L2 sees a run of
+// neighbouring blocks, whose rows and face velocities they share.
 __device__ __forceinline__ int xcd_item(int b, int per) { return (b & 7) * per + (b >> 3); }
 __device__ __forceinline__ void flat_item(const FlatGrid &f, int L, int &n, int &blk, int &k0) {
     n = L & 1;
@@ -73,9 +74,12 @@ __device__ __forceinline__ D2 ld2(const double *plane, uint32_t off) {
 __device__ __forceinline__ uint32_t ldf2(const uint8_t *plane, uint32_t off) {
     return *reinterpret_cast<const licom_u16 *>(plane + off);
 }
-// Stores of the cells that a0 and a1 mark.  Non-temporal: nothing on this
-// path reads them again before the caches have turned over (k_update 5.22 ->
-// 5.02 ms at 1800 x 1151 x 55, 98 -> 82 us at 225 x 145 x 55).
+// Stores of the cells that a0 and a1 mark.  Non-temporal: on a large grid
+// nothing reads them again before the caches have turned over (k_update 5.22 ->
+// 5.02 ms at 1800 x 1151 x 55).  On a small one k_solve reads ori, one of them,
+// from the caches; with ori alone stored plainly k_update takes 22.6 us in
+// place of 21.3 at 128 x 96 x 30, 121 in place of 113 at 360 x 218 x 30, and the
+// solve the same to 2 us, so ori goes the same way.
 __device__ __forceinline__ void st2(double *plane, uint32_t off, const double (&x)[2], bool a0, bool a1) {
     char *p = reinterpret_cast<char *>(plane) + off;
     if (a0 && a1) {
@@ -112,8 +116,10 @@ __device__ __forceinline__ void march_levels(int k0, int k1, int km, F &&level) 
     if (k < k1) level(std::integral_constant<int, 2>{}, k);
 }
 
-// Byte offsets of the lane's cells and of those dj rows away, kept inside
-// the plane (a lane that owns a cell never has its offsets clamped).
+// First of the lane's cells, or of those some rows away, kept inside the
+// plane.  What is read for a cell in columns 1..imt-2 is never clamped; a lane
+// that owns the last cell of row jmt-2 (k_flags with an odd cell count) has the
+// row below clamped, and the flag it stores there is one that nothing reads.
 __device__ __forceinline__ int clamp_cell(int p, int n2) { return min(max(p, 0), n2 - 2); }
 
 // Keeps the compiler from forming plane + offset once per array outside the

@@ -67,7 +67,7 @@ struct licom_ctx {
     // licomqice [jmt][imt] (device) written by steps with LICOM_STEP_ICESNOW
     double *qice = nullptr;
     // tspas limiter flags [2][km][jmt][imt] (device, 1 byte) written by the
-    // FP64 update and the mixed k-march when set (licom_tracer_set_flag_output)
+    // FP64 and the mixed update when set (licom_tracer_set_flag_output)
     uint8_t *flags_out = nullptr;
     licom::KGrid g{};
     licom::KPar kp{};

@@ -97,10 +97,15 @@ extern "C" int licom_tracer_step_noalloc(licom_ctx *c, const licom_fields *f, co
     if (int rc = plan_step(c, f, flags, split, "licom_tracer_step_noalloc")) return rc;
     const uintptr_t al = reinterpret_cast<uintptr_t>(f->at) | reinterpret_cast<uintptr_t>(f->atb) |
                          reinterpret_cast<uintptr_t>(f->ws) | reinterpret_cast<uintptr_t>(f->akt);
-    if ((flags & LICOM_STEP_STAGED) || c->imt % 2 != 0 || (al & 15) != 0) {
-        set_error("licom_tracer_step_noalloc runs the fused kernels only: it needs an even imt, "
-                  "16-byte aligned at/atb/ws/akt, no LICOM_STEP_STAGED and not ICESNOW with "
-                  "VTL_SCRATCH");
+    if (flags & LICOM_STEP_STAGED) {
+        set_error("licom_tracer_step_noalloc runs the fused kernels only: no LICOM_STEP_STAGED and "
+                  "no ICESNOW with VTL_SCRATCH");
+        return LICOM_ENOTSUP;
+    }
+    // this entry point's own limits: the kernels take any imt and alignment
+    if (c->imt % 2 != 0 || (al & 15) != 0) {
+        set_error("licom_tracer_step_noalloc takes an even imt and 16-byte aligned at/atb/ws/akt only "
+                  "(licom_tracer_step takes any)");
         return LICOM_ENOTSUP;
     }
     Scratch s;

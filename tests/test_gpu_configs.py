@@ -6,8 +6,7 @@ for the batch engine and the request loop, against each member run alone.
   0.1 deg benchmark runs), on the default and the wide-grid launch shape
 * LICOM_STEP_VTL_SCRATCH on a convecting case: vtl holds tracer_'s S,
   before convadj (tracer.cpp:1880-1893, convadj.cpp)
-* the mixed form on a grid that does not tile into the mixed march's 32x6
-  tiles (partial tiles on both axes)
+* the mixed form on a grid whose cells end in a partial run of the update
 * the mixed form at the full 3600x2302x55 size: T/S content conservation and
   heat drift against the FP64 form
 * the 64-member ensemble of the benchmark (domains and seeds of its
@@ -56,7 +55,7 @@ def max_err(case, a, b):
 # ------------------------------------------------------------ FP64 km = 55
 @pytest.mark.parametrize("nx,ny,tag", [(128, 96, "default launch"), (520, 24, "wide-grid launch")])
 def test_km55_fp64_step_with_convadj_bitwise(nx, ny, tag, need_gpu):
-    """k_prelude_col<55>, the k-march and k_solve<55, double, double> with
+    """k_prelude_col<55>, k_flags, k_update and k_solve<55, double, double> with
     convadj (no icesnow): the kernels of the 0.1 deg benchmark, with its
     del4 mixing and 600 s step."""
     announce(f"fp64 km55 del4 dt=600 x2, {nx}x{ny} ({tag})")
@@ -115,9 +114,10 @@ def test_vtl_scratch_without_convadj(need_gpu):
 
 # ---------------------------------------------------------- mixed, ragged
 def test_mixed_partial_tiles_against_oracle(need_gpu):
-    """100x50 columns: the mixed march's 32x6 tiles end in partial tiles on
-    both axes (100 = 3*32 + 4, 50 = 8*6 + 2)."""
-    announce("mixed 100x50x30 1 step vs oracle (partial tiles)")
+    """100x50 columns: the last of the update's workgroups (4 runs of 124
+    cells over rows of 104) and of the prelude's 64-column blocks are part
+    full."""
+    announce("mixed 100x50x30 1 step vs oracle (partial runs)")
     case = ls.make_case("C1", nx=100, ny=50, km=30, seed=14, depth_min=-1000.0, sigma=2.0)
     o = orc.Oracle(case)
     st = case.copy_state()
@@ -130,13 +130,13 @@ def test_mixed_partial_tiles_against_oracle(need_gpu):
     eT, eS = max_err(case, gs["at"], st["at"])
     print(f"[mixed 100x50] max|dT| {eT:.3e} K, max|dS| {eS:.3e} psu", flush=True)
     assert eT <= 1e-6 and eS <= 1e-6
-    # the tile edges: the last partial column and row of tiles
+    # the last columns apart: the end of the prelude's partial blocks
     for k in ("ax", "ay", "az", "tend"):
         a, b = inner(gd[k]), inner(od[k])
         scale = np.abs(b).max()
         err = np.abs(a - b).max() / scale
         edge = np.abs(a[..., :, 96:] - b[..., :, 96:]).max() / scale
-        print(f"  {k}: rel {err:.3e} (last partial tile column {edge:.3e})", flush=True)
+        print(f"  {k}: rel {err:.3e} (last columns {edge:.3e})", flush=True)
         assert err <= 1e-4, k
 
 

@@ -157,8 +157,8 @@ def test_derived_masks_and_coefficients_bitwise(need_gpu):
 
 def test_wide_grid_bitwise(need_gpu):
     """520 columns: the solve takes one 128-column row per workgroup (the
-    launch used for the 0.1 deg grid) and the k-march tiles wrap 33 times
-    along i; two steps with del4, bit for bit."""
+    launch used for the 0.1 deg grid) and a row holds more than four of the
+    update's 124-cell runs; two steps with del4, bit for bit."""
     announce("two steps 520x24x12 del4 (wide-grid launch shapes)")
     case = ls.make_case("C1", nx=520, ny=24, km=12, seed=21, hmix=4, ah=-1.0e10)
     case.name = "C1-wide"

@@ -1,6 +1,6 @@
 """GPU parity of the centered and flux advection schemes (advection_tracer_1,
 tracer.cpp:120-289, selected by adv_tracer at tracer.cpp:1712-1714) against
-the oracle, bit for bit: the fused k-march and the per-stage kernels, del2
+the oracle, bit for bit: the fused k_update and the per-stage kernels, del2
 and del4, with convadj and the side effects; the centered scheme's ax/ay/az
 accumulate over the steps (divided by nss), the flux scheme leaves them
 alone.  The mixed form and batches refuse both schemes."""
@@ -53,7 +53,7 @@ def test_scheme_steps_bitwise(adv, hmix, staged, need_gpu):
 
 
 def test_centered_wide_grid_bitwise(need_gpu):
-    """Tiles with partial edges and the 128-column solve rows."""
+    """The 128-column solve rows, and runs of cells that end in mid-row."""
     case = ls.make_case("C1", nx=530, ny=26, km=12, seed=21, depth_min=-2500.0, sigma=2.0)
     case.params["adv"] = ls.ADV_CENTERED
     case.params["nss"] = 1
