@@ -23,6 +23,7 @@ struct FlatGrid {
     int first, last;  // cells [first, last) of the plane
     int nch, kc;      // chunks of a column, levels per chunk
     int total, per;   // workgroups, and workgroups per XCD
+    bool apart;       // all of one tracer before the other (update_grid)
 };
 
 // Whole columns, where those give the 256 CUs four workgroups each (smaller
@@ -37,17 +38,35 @@ inline FlatGrid flat_grid(int first, int last, int km, int want = 1024) {
     const int kc = std::max((km + nch - 1) / nch, 2);
     nch = (km + kc - 1) / kc;
     const int total = 2 * nb * nch;
-    return FlatGrid{first, last, nch, kc, total, (total + 7) / 8};
+    return FlatGrid{first, last, nch, kc, total, (total + 7) / 8, false};
 }
 
-// Block -> (tracer, chunk, block of the plane): the two tracers of one place,
-// then its chunks, run next to each other, and the hardware's round-robin deal
-// of blocks to the eight XCDs is undone, so that each XCD's L2 sees a run of
-// neighbouring blocks, whose rows and face velocities they share.
+// The update's grid.  Where its plane fills the chip with whole columns, all
+// workgroups of T come before those of S: side by side, the two tracers have
+// twice as many planes open at a time, which costs more there than the face
+// velocities and metrics that they could share (k_update_mx at 3600 x 2302 x 55
+// 15.8 -> 14.6 ms, with which the mixed step takes 42.1 ms and not 43.2; at
+// 1800 x 1151 x 55 3.64 -> 3.57; k_update 19.0 -> 18.2 and 5.10 -> 4.96; at
+// 600 x 440 x 55 either way the same).  On small planes, which the L2s hold, it
+// is the other way round (k_update_mx at 96 x 64 x 55: 13.4 us side by side, 14.4
+// apart; k_update at 128 x 96 x 30: 21.3, 23), and for the flags on every plane
+// (k_flags_mx at 3600 x 2302 x 55: 4.46, 4.68 ms).
+inline FlatGrid update_grid(int imt, int jmt, int km, int want = 1024) {
+    FlatGrid f = flat_grid(2 * imt, (jmt - 2) * imt, km, want);
+    f.apart = f.total / f.nch >= 1024;
+    return f;
+}
+
+// Block -> (tracer, chunk, block of the plane): the two tracers of one place
+// (unless they are kept apart), then its chunks, run next to each other, and
+// the hardware's round-robin deal of blocks to the eight XCDs is undone, so
+// that each XCD's L2 sees a run of neighbouring blocks, whose rows and face
+// velocities they share.
 __device__ __forceinline__ int xcd_item(int b, int per) { return (b & 7) * per + (b >> 3); }
 __device__ __forceinline__ void flat_item(const FlatGrid &f, int L, int &n, int &blk, int &k0) {
-    n = L & 1;
-    const int h = L >> 1;
+    const int half = f.total >> 1;
+    n = f.apart ? L >= half : L & 1;
+    const int h = f.apart ? L - n * half : L >> 1;
     blk = h / f.nch;
     k0 = (h - blk * f.nch) * f.kc;
 }

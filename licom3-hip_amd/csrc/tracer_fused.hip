@@ -190,10 +190,10 @@ __global__ __launch_bounds__(256) void k_prelude_col(KGrid g, KPar p, const doub
 // --------------------------------------------------- limiter flags and update
 // Replaces a march of 16 x 12 tiles whose planes a fourth wave staged in LDS
 // (two barriers a level, two workgroups per CU: bound by the latency of its
-// level loop, 7.03 ms at 1800 x 1151 x 55, 71 us at 128 x 96 x 30; now 6.65 ms
+// level loop, 7.03 ms at 1800 x 1151 x 55, 71 us at 128 x 96 x 30; now 6.5 ms
 // and 32 us, k_flags bound by its ~200 FP64 instructions a cell and k_update
-// by its 11 + 8 planes of HBM traffic, 4.2 TB/s; at 3600 x 2302 x 55 the pair
-// takes what the march did, 27 ms).  Neither kernel carries anything from one
+// by its 11 + 8 planes of HBM traffic, 4.2 TB/s; at 3600 x 2302 x 55 it
+// was 26.5 ms and is 24.8).  Neither kernel carries anything from one
 // level to the next but values it has already loaded, so a column is cut into
 // chunks of levels and every (chunk, run of cells, tracer) is a workgroup of
 // its own.  Runs of cells and chunks: tracer_cells.h.
@@ -620,7 +620,7 @@ void launch_update(licom_ctx *ctx, const licom_fields *f, const licom_diag *d, c
     a.dz = d ? d->dz : nullptr;
     a.pen = d ? d->penetrate : nullptr;
     a.flags_out = ctx->flags_out;
-    const FlatGrid fg = flat_grid(2 * g.imt, (g.jmt - 2) * g.imt, g.km);
+    const FlatGrid fg = update_grid(g.imt, g.jmt, g.km);
     auto kern = ctx->kp.hmix == LICOM_HMIX_DEL4 ? k_update<ADV, true> : k_update<ADV, false>;
     kern<<<8 * fg.per, 256, 0, st>>>(g, ctx->kp, f->at, f->atb, f->akt, s.uw, s.vs, f->ws, s.flags, s.ori, g.odzp,
                                      g.odzt, g.pen, a, fg);

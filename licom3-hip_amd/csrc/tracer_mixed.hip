@@ -761,7 +761,7 @@ int launch_step_mixed(licom_ctx *ctx, const licom_fields_mixed *f, const licom_d
             k_flags_mx<<<8 * ff.per, 256, 0, st>>>(g, ctx->kp.dts, a, ff);
         }
         Timer t(ctx, "k_update");
-        const FlatGrid fu = flat_grid(2 * g.imt, (g.jmt - 2) * g.imt, g.km);
+        const FlatGrid fu = update_grid(g.imt, g.jmt, g.km);
         if (ctx->kp.hmix == LICOM_HMIX_DEL4) k_update_mx<true><<<8 * fu.per, 256, 0, st>>>(g, ctx->kp, a, fu);
         else k_update_mx<false><<<8 * fu.per, 256, 0, st>>>(g, ctx->kp, a, fu);
     }
@@ -1388,7 +1388,7 @@ extern "C" int licom_batch_create(licom_ctx *const *members, const licom_fields_
         // this member's share of the workgroups that fill the chip
         const int want = (int)(1024.0 * (double)n2 / cells) + 1;
         d.ff = flat_grid(imt, (jmt - 1) * imt, km, want);
-        d.fu = flat_grid(2 * imt, (jmt - 2) * imt, km, want);
+        d.fu = update_grid(imt, jmt, km, want);
         d.side_vec = ((reinterpret_cast<uintptr_t>(f.utf) | reinterpret_cast<uintptr_t>(f.vtf)) & 15) == 0 &&
                      n3 % 4 == 0;
         d.side_blocks = (int)(((d.side_vec ? n3 / 4 : n3) + 255) / 256);
