@@ -28,10 +28,10 @@ struct FlatGrid {
 
 // Whole columns, where those give the 256 CUs four workgroups each (smaller
 // chunks read the levels around them again: at 1800 x 1151 x 55 chunks of 55,
-// 28, 14 and 7 levels take 6.65, 6.69, 6.79 and 7.16 ms for both FP64 kernels),
-// and otherwise as many chunks as that takes (want: its share of the 1024
-// workgroups), of two levels at least.  A plane has five rows or more, so it
-// is never without cells.
+// 28, 14 and 7 levels took 6.65, 6.69, 6.79 and 7.16 ms for both FP64 kernels,
+// their tracers side by side), and otherwise as many chunks as that takes
+// (want: its share of the 1024 workgroups), of two levels at least.  A plane
+// has five rows or more, so it is never without cells.
 inline FlatGrid flat_grid(int first, int last, int km, int want = 1024) {
     const int nb = (last - first + 4 * kWaveCells - 1) / (4 * kWaveCells);
     int nch = std::max((want + 2 * nb - 1) / (2 * nb), 1);
